@@ -3,7 +3,9 @@
 // hand-written kernels.  Every matrix product runs on the matrix cores
 // (v_mfma_f32_16x16x4_f32, one 16x16 tile per workgroup, K split across its
 // waves); bias, ReLU, the masked MSE gradient and Adam are elementwise
-// kernels.  No reference counterpart.
+// kernels.  A training step of a network that fits one workgroup's LDS (the
+// cost model's does) is two launches instead: mlp_step_kernel and
+// mlp_update_kernel.  No reference counterpart.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -131,6 +133,233 @@ __global__ __launch_bounds__(256) void adam_kernel(float *__restrict__ p, const 
   p[i] -= lr_t * mi / (sqrtf(vi) + eps);
 }
 
+// ---- a training step in two launches --------------------------------------
+// Layer by layer a step is 16 launches of 2-6 us each for 25 MFLOP, and the
+// loss read back every epoch drains the queue: 113 us per epoch at 695 rows
+// of 24 -> 64 -> 64 -> 6, all of it latency.  Here the whole network sits in
+// one workgroup's LDS (63 KB) and a workgroup carries a tile of 16 rows
+// through the forward pass, the loss and the backward pass without leaving
+// it; its parts of the weight gradients stay in MFMA accumulators over all its
+// tiles and are stored once.  A second launch sums the workgroups' parts and
+// applies Adam: 9.5 + 3.8 us per epoch at 695 rows (44 workgroups), bound by
+// the chain of loads, products and barriers, and 20 epochs as one call 2216 ->
+// 350 us.
+constexpr uint32_t kStepWidth = 64;   // most inputs and hidden units
+constexpr uint32_t kStepOutputs = 16; // most outputs
+constexpr uint32_t kStepRows = 16;    // rows of a tile (one MFMA tile's)
+// at most one workgroup per CU: beyond 4096 rows a workgroup takes several
+// tiles, so the gradient parts stay under 256 x the parameters
+constexpr uint32_t kStepBlocks = 256;
+// LDS row stride: lanes l of an operand read word (l % 16) * 68 + l / 16, 64
+// different banks
+constexpr uint32_t kStepStride = kStepWidth + 4;
+
+struct MlpShape {
+  uint32_t I, H, O;
+  __host__ __device__ uint32_t b1() const { return H * I; }
+  __host__ __device__ uint32_t w2() const { return b1() + H; }
+  __host__ __device__ uint32_t b2() const { return w2() + H * H; }
+  __host__ __device__ uint32_t w3() const { return b2() + H; }
+  __host__ __device__ uint32_t b3() const { return w3() + O * H; }
+  __host__ __device__ uint32_t params() const { return b3() + O; }
+};
+
+// dst[row][col] (stride kStepStride) = src[row][col], zero outside rows x cols
+template <uint32_t ROWS>
+__device__ __forceinline__ void step_load(float *dst, const float *__restrict__ src, uint32_t rows,
+                                          uint32_t cols, uint32_t t) {
+  float v[ROWS / 4];
+#pragma unroll
+  for (uint32_t i = 0; i < ROWS / 4; ++i) {
+    const uint32_t r = (t >> 6) + 4 * i, c = t & 63u;
+    v[i] = (r < rows && c < cols) ? src[size_t(r) * cols + c] : 0.f;
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < ROWS / 4; ++i) dst[((t >> 6) + 4 * i) * kStepStride + (t & 63u)] = v[i];
+}
+
+// acc += A B over k < K (a multiple of 4), A(i,k) = a[i * sai + k * sak] and
+// B(k,j) = b[k * sbk + j * sbj] in LDS, zero-padded to whole tiles
+template <uint32_t K>
+__device__ __forceinline__ v4f step_mfma(v4f acc, const float *a, uint32_t sai, uint32_t sak,
+                                         const float *b, uint32_t sbk, uint32_t sbj,
+                                         uint32_t lane) {
+  const float *pa = a + (lane & 15u) * sai + (lane >> 4) * sak;
+  const float *pb = b + (lane & 15u) * sbj + (lane >> 4) * sbk;
+  // two chains, so that one product's latency hides the other's
+  v4f odd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (uint32_t k = 0; k < K; k += 8) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[k * sak], pb[k * sbk], acc, 0, 0, 0);
+    if (k + 4 < K)
+      odd = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[(k + 4) * sak], pb[(k + 4) * sbk], odd, 0, 0,
+                                                 0);
+  }
+  return acc + odd;
+}
+
+// the sum of a C tile's column, in every lane of the column
+__device__ __forceinline__ float step_colsum(const float *v) {
+  float s = (v[0] + v[1]) + (v[2] + v[3]);
+  s += __shfl_xor(s, 16);
+  s += __shfl_xor(s, 32);
+  return s;
+}
+
+// Forward, loss and backward of the rows of tiles blockIdx.x, + gridDim.x,
+// ...; part[blockIdx.x][params] gets the workgroup's sums of the gradients,
+// loss_part[blockIdx.x] its sum of mask (y - t)^2.  Four waves; wave w owns
+// columns 16 w .. 16 w + 15 of each layer.  Rows past the end carry zeros:
+// their gradients are set to zero whatever the weights are.  IN: the inputs
+// rounded up to 32 or 64 (half the first layer's products at 24 inputs).
+template <uint32_t IN>
+__global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *__restrict__ p,
+                                                       const float *__restrict__ X,
+                                                       const float *__restrict__ T,
+                                                       const float *__restrict__ mask,
+                                                       uint32_t rows, float inv_count,
+                                                       float *__restrict__ part,
+                                                       float *__restrict__ loss_part) {
+  constexpr uint32_t S = kStepStride, W = kStepWidth;
+  __shared__ float w1[W * S], w2[W * S], w3[kStepOutputs * S];
+  __shared__ float xs[kStepRows * S], h1[kStepRows * S], h2[kStepRows * S];
+  __shared__ float d1[kStepRows * S], d2[kStepRows * S], dy[kStepRows * 20];
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6, r = lane & 15u, q = lane >> 4;
+  const uint32_t col = 16 * w + r; // this lane's column of a hidden layer
+  step_load<W>(w1, p, s.H, s.I, t);
+  step_load<W>(w2, p + s.w2(), s.H, s.H, t);
+  step_load<kStepOutputs>(w3, p + s.w3(), s.O, s.H, t);
+  const float b1 = col < s.H ? p[s.b1() + col] : 0.f, b2 = col < s.H ? p[s.b2() + col] : 0.f;
+  const uint32_t yr = t >> 4, yc = t & 15u; // this thread's output value
+  const float b3 = yc < s.O ? p[s.b3() + yc] : 0.f;
+  const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  v4f g1[IN / 16], g2[4] = {zero, zero, zero, zero}, g3 = zero;
+#pragma unroll
+  for (uint32_t j = 0; j < IN / 16; ++j) g1[j] = zero;
+  float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, loss = 0.f;
+  for (uint32_t row0 = blockIdx.x * kStepRows; row0 < rows; row0 += gridDim.x * kStepRows) {
+    const uint32_t n = min(kStepRows, rows - row0);
+    step_load<kStepRows>(xs, X + size_t(row0) * s.I, n, s.I, t);
+    const size_t yi = size_t(row0 + yr) * s.O + yc;
+    const bool live = yr < n && yc < s.O;
+    const float target = live ? T[yi] : 0.f, weight = live ? (mask ? mask[yi] : 1.f) : 0.f;
+    __syncthreads();
+    v4f a = step_mfma<IN>(zero, xs, S, 1, w1 + 16 * w * S, 1, S, lane);
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      const float z = a[v] + b1;
+      h1[(4 * q + v) * S + col] = z > 0.f ? z : 0.f;
+    }
+    __syncthreads();
+    a = step_mfma<W>(zero, h1, S, 1, w2 + 16 * w * S, 1, S, lane);
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      const float z = a[v] + b2;
+      h2[(4 * q + v) * S + col] = z > 0.f ? z : 0.f;
+    }
+    __syncthreads();
+    // the one output tile: each wave a quarter of its sum, through d1
+    a = step_mfma<W / 4>(zero, h2 + 16 * w, S, 1, w3 + 16 * w, 1, S, lane);
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) d1[w * 256 + (4 * q + v) * 16 + r] = a[v];
+    __syncthreads();
+    const float y = ((d1[t] + d1[256 + t]) + (d1[512 + t] + d1[768 + t])) + b3;
+    const float e = live ? (y - target) * weight : 0.f;
+    if (live) loss += e * (y - target);
+    dy[yr * 20 + yc] = 2.f * e * inv_count;
+    __syncthreads();
+    a = step_mfma<kStepOutputs>(zero, dy, 20, 1, w3 + 16 * w, S, 1, lane);
+    float dz[4];
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      const uint32_t row = 4 * q + v;
+      dz[v] = (row < n && h2[row * S + col] > 0.f) ? a[v] : 0.f;
+      d2[row * S + col] = dz[v];
+    }
+    gb2 += step_colsum(dz);
+    g3 = step_mfma<kStepRows>(g3, dy, 1, 20, h2 + 16 * w, S, 1, lane);
+    if (w == 0) gb3 += step_colsum((const float[4]){dy[(4 * q) * 20 + r], dy[(4 * q + 1) * 20 + r],
+                                                    dy[(4 * q + 2) * 20 + r],
+                                                    dy[(4 * q + 3) * 20 + r]});
+    __syncthreads();
+    a = step_mfma<W>(zero, d2, S, 1, w2 + 16 * w, S, 1, lane);
+#pragma unroll
+    for (uint32_t v = 0; v < 4; ++v) {
+      const uint32_t row = 4 * q + v;
+      dz[v] = (row < n && h1[row * S + col] > 0.f) ? a[v] : 0.f;
+      d1[row * S + col] = dz[v];
+    }
+    gb1 += step_colsum(dz);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j)
+      g2[j] = step_mfma<kStepRows>(g2[j], d2 + 16 * w, 1, S, h1 + 16 * j, S, 1, lane);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < IN / 16; ++j)
+      g1[j] = step_mfma<kStepRows>(g1[j], d1 + 16 * w, 1, S, xs + 16 * j, S, 1, lane);
+    __syncthreads(); // xs, h1 and d1 are free for the next tile
+  }
+  float *g = part + size_t(blockIdx.x) * s.params();
+#pragma unroll
+  for (uint32_t v = 0; v < 4; ++v) {
+    const uint32_t row = 16 * w + 4 * q + v; // g1, g2: this wave's 16 rows
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t c = 16 * j + r;
+      if (j < IN / 16 && row < s.H && c < s.I) g[row * s.I + c] = g1[j][v];
+      if (row < s.H && c < s.H) g[s.w2() + row * s.H + c] = g2[j][v];
+    }
+    if (4 * q + v < s.O && col < s.H) g[s.w3() + (4 * q + v) * s.H + col] = g3[v];
+  }
+  if (q == 0 && col < s.H) g[s.b1() + col] = gb1, g[s.b2() + col] = gb2;
+  if (w == 0 && q == 0 && r < s.O) g[s.b3() + r] = gb3;
+#pragma unroll
+  for (uint32_t o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+  if (lane == 0) xs[w] = loss;
+  __syncthreads();
+  if (t == 0) loss_part[blockIdx.x] = (xs[0] + xs[1]) + (xs[2] + xs[3]);
+}
+
+// Sums the workgroups' gradient parts (in FP64, four slices of them per
+// parameter) and either applies Adam or, with grad, stores the sums; the last
+// workgroup also sums the loss.  64 parameters per workgroup.
+__global__ __launch_bounds__(256) void mlp_update_kernel(
+    float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
+    const float *__restrict__ part, const float *__restrict__ loss_part, uint32_t n,
+    uint32_t parts, float lr_t, float b1, float b2, float eps, float wd, float count,
+    float *__restrict__ grad, float *__restrict__ loss) {
+  __shared__ double sum[256];
+  const uint32_t t = threadIdx.x, i = blockIdx.x * 64u + (t & 63u);
+  const uint32_t at = min(i, n - 1);
+  const float pi = p[at], m0 = m[at], v0 = v[at];
+  double acc = 0.0;
+#pragma unroll 8
+  for (uint32_t j = t >> 6; j < parts; j += 4) acc += double(part[size_t(j) * n + at]);
+  sum[t] = acc;
+  __syncthreads();
+  if (t < 64 && i < n) {
+    const float g0 = float((sum[t] + sum[t + 64]) + (sum[t + 128] + sum[t + 192]));
+    if (grad) {
+      grad[i] = g0;
+    } else {
+      const float gi = g0 + wd * pi;
+      const float mi = b1 * m0 + (1.f - b1) * gi;
+      const float vi = b2 * v0 + (1.f - b2) * gi * gi;
+      m[i] = mi, v[i] = vi;
+      p[i] = pi - lr_t * mi / (sqrtf(vi) + eps);
+    }
+  }
+  if (!loss || blockIdx.x + 1 != gridDim.x) return;
+  __syncthreads();
+  sum[t] = t < parts ? double(loss_part[t]) : 0.0; // parts <= kStepBlocks
+  __syncthreads();
+  for (uint32_t o = 128; o > 0; o >>= 1) {
+    if (t < o) sum[t] += sum[t + o];
+    __syncthreads();
+  }
+  if (t == 0) *loss = float(sum[0] / count);
+}
+
 uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
 // C (MxN) = op(A) op(B) through strides; see gemm_mfma_kernel
@@ -170,6 +399,10 @@ struct fot_mlp {
   uint32_t cap = 0;
   float *X = nullptr, *H1 = nullptr, *H2 = nullptr, *Y = nullptr, *T = nullptr, *Mk = nullptr;
   float *dY = nullptr, *dH2 = nullptr, *dH1 = nullptr, *part = nullptr;
+  // two-launch training steps: gradient and loss parts of the workgroups, the
+  // epochs' losses
+  float *gpart = nullptr, *lpart = nullptr, *losses = nullptr;
+  uint32_t gcap = 0, lcap = 0;
   uint64_t step = 0;
   std::vector<void *> owned;
 
@@ -250,6 +483,43 @@ struct fot_mlp {
       for (float x : h) acc += x;
       *loss = float(acc / count);
     }
+    return FOT_OK;
+  }
+  // Whether a training step runs as two launches: the network fits the LDS of
+  // mlp_step_kernel.  Wider networks go layer by layer.
+  bool fits_step() const { return I <= kStepWidth && H <= kStepWidth && O <= kStepOutputs; }
+  fot_status resize(float **q, uint32_t *have, uint32_t want, size_t each) {
+    if (want <= *have) return FOT_OK;
+    if (*q) {
+      owned.erase(std::find(owned.begin(), owned.end(), static_cast<void *>(*q)));
+      (void)hipFree(*q);
+      *q = nullptr;
+      *have = 0;
+    }
+    if (fot_status st = alloc(q, want * each)) return st;
+    *have = want;
+    return FOT_OK;
+  }
+  fot_status reserve_step(uint32_t rows, uint32_t epochs) {
+    fot_status st;
+    if (!lpart && (st = alloc(&lpart, kStepBlocks))) return st;
+    if ((st = resize(&gpart, &gcap, step_blocks(rows), nparam))) return st;
+    return resize(&losses, &lcap, epochs, 1);
+  }
+  static uint32_t step_blocks(uint32_t rows) { return std::min(cdiv(rows, kStepRows), kStepBlocks); }
+  // One step over the loaded rows (reserve_step first): Adam with lr_t, or the
+  // gradient into g when `gradient`; the loss into losses[e] when wanted.
+  fot_status fused_step(uint32_t rows, bool masked, float count, bool gradient, float lr_t,
+                        float b1, float b2, float eps, float wd, bool want_loss, uint32_t e,
+                        hipStream_t s) {
+    const uint32_t nb = step_blocks(rows), n = uint32_t(nparam);
+    hipLaunchKernelGGL(I <= 32 ? mlp_step_kernel<32> : mlp_step_kernel<64>, dim3(nb), dim3(256), 0,
+                       s, (MlpShape{I, H, O}), p, X, T, masked ? Mk : nullptr, rows, 1.f / count,
+                       gpart, lpart);
+    hipLaunchKernelGGL(mlp_update_kernel, dim3(cdiv(n, 64)), dim3(256), 0, s, p, m, v, gpart,
+                       lpart, n, nb, lr_t, b1, b2, eps, wd, count, gradient ? g : nullptr,
+                       want_loss ? losses + e : nullptr);
+    FOT_HIP(hipGetLastError());
     return FOT_OK;
   }
   fot_status load_rows(const float *x, const float *t, const float *mask, uint32_t rows) {
@@ -432,9 +702,17 @@ static fot_status fot_mlp_loss_grad_impl(fot_mlp *mlp, const float *x, const flo
     return fail(FOT_ERR_INVALID_ARGUMENT, "null argument");
   fot_status st;
   if ((st = mlp->load_rows(x, t, mask, rows))) return st;
-  if ((st = mlp->forward(rows, nullptr))) return st;
   const float count = mask_count(mask, size_t(rows) * mlp->O);
-  if ((st = mlp->backward(rows, mask != nullptr, count, loss, nullptr))) return st;
+  if (mlp->fits_step()) {
+    if ((st = mlp->reserve_step(rows, 1))) return st;
+    if ((st = mlp->fused_step(rows, mask != nullptr, count, true, 0.f, 0.f, 0.f, 0.f, 0.f, true, 0,
+                              nullptr)))
+      return st;
+    FOT_HIP(hipMemcpy(loss, mlp->losses, sizeof(float), hipMemcpyDeviceToHost));
+  } else {
+    if ((st = mlp->forward(rows, nullptr))) return st;
+    if ((st = mlp->backward(rows, mask != nullptr, count, loss, nullptr))) return st;
+  }
   FOT_HIP(hipMemcpy(grad, mlp->g, mlp->nparam * sizeof(float), hipMemcpyDeviceToHost));
   return FOT_OK;
 }
@@ -454,22 +732,35 @@ static fot_status fot_mlp_train_impl(fot_mlp *mlp, const float *x, const float *
   if ((st = mlp->load_rows(x, t, mask, rows))) return st;
   const float count = mask_count(mask, size_t(rows) * mlp->O);
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const bool fused = mlp->fits_step();
+  if (fused && (st = mlp->reserve_step(rows, loss_per_epoch ? epochs : 0))) return st;
   for (uint32_t e = 0; e < epochs; ++e) {
-    if ((st = mlp->forward(rows, nullptr))) return st;
-    float l = 0;
-    if ((st = mlp->backward(rows, mask != nullptr, count, loss_per_epoch ? &l : nullptr, nullptr)))
-      return st;
-    if (loss_per_epoch) loss_per_epoch[e] = l;
+    if (!fused) {
+      if ((st = mlp->forward(rows, nullptr))) return st;
+      float l = 0;
+      if ((st = mlp->backward(rows, mask != nullptr, count, loss_per_epoch ? &l : nullptr,
+                              nullptr)))
+        return st;
+      if (loss_per_epoch) loss_per_epoch[e] = l;
+    }
     ++mlp->step;
     const double c1 = 1.0 - std::pow(double(b1), double(mlp->step));
     const double c2 = 1.0 - std::pow(double(b2), double(mlp->step));
     const float lr_t = float(lr * std::sqrt(c2) / c1);
+    if (fused) {
+      if ((st = mlp->fused_step(rows, mask != nullptr, count, false, lr_t, b1, b2, eps,
+                                weight_decay, loss_per_epoch != nullptr, e, nullptr)))
+        return st;
+      continue;
+    }
     hipLaunchKernelGGL(adam_kernel, dim3(cdiv(uint32_t(mlp->nparam), 256)), dim3(256), 0, nullptr,
                        mlp->p, mlp->g, mlp->m, mlp->v, uint32_t(mlp->nparam), lr_t, b1, b2, eps,
                        weight_decay);
     FOT_HIP(hipGetLastError());
   }
   FOT_HIP(hipDeviceSynchronize());
+  if (fused && loss_per_epoch && epochs)
+    FOT_HIP(hipMemcpy(loss_per_epoch, mlp->losses, sizeof(float) * epochs, hipMemcpyDeviceToHost));
   return FOT_OK;
 }
 extern "C" fot_status fot_mlp_train(fot_mlp *mlp, const float *x, const float *t,

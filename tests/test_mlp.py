@@ -95,3 +95,42 @@ def test_mlp_training_fits_a_smooth_target(gpu):
     # the trained parameters reproduce the reported loss through the oracle
     lr_, _ = MO.loss_grad(net.get_params().astype(np.float64), x, t, None, 24, 64, 6)
     assert lr_ < 0.1 * losses[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_in,hidden,n_out,rows,masked", [
+    (1, 1, 1, 1, False), (24, 64, 6, 16, True), (24, 64, 6, 17, False), (33, 40, 7, 95, True),
+    (64, 64, 16, 4096, True), (24, 64, 6, 4113, True), (32, 5, 16, 300, False),
+    (24, 65, 6, 50, True), (65, 16, 3, 50, False), (8, 16, 17, 50, True)])
+def test_mlp_step_at_tile_edges(gpu, n_in, hidden, n_out, rows, masked):
+    """Gradient and a step of training at the edges of the one-workgroup
+    network's tiles (rows of 16, widths of 32 and 64, 16 outputs, more rows
+    than workgroups take at once) and just beyond, where the layers run one
+    by one."""
+    from cuda_fot_amd.mlp import MLP
+    rng = np.random.default_rng(n_in * 1000 + rows)
+    net = MLP(n_in, hidden, n_out, seed=5)
+    p = net.get_params().astype(np.float64)
+    x = rng.normal(size=(rows, n_in)).astype(np.float32)
+    t = rng.normal(size=(rows, n_out)).astype(np.float32)
+    m = (rng.random((rows, n_out)) > 0.2).astype(np.float32) if masked else None
+    loss, g = net.loss_grad(x, t, m)
+    lr, gr = MO.loss_grad(p, x, t, m, n_in, hidden, n_out)
+    assert abs(loss - lr) <= 1e-5 * lr
+    k = 0
+    for shape in [(hidden, n_in), (hidden,), (hidden, hidden), (hidden,), (n_out, hidden),
+                  (n_out,)]:
+        n = int(np.prod(shape))
+        # FP32 sums of up to 4113 rows: 4113 * 2^-24 = 2.5e-4 of the sum of
+        # magnitudes at worst
+        np.testing.assert_allclose(g[k:k + n], gr[k:k + n],
+                                   atol=2.5e-4 * np.abs(gr[k:k + n]).max() + 1e-12, rtol=0)
+        k += n
+    losses = net.train(x, t, m, epochs=3, lr=1e-3, weight_decay=0.1)
+    assert losses[0] == loss
+    # Adam's first steps move a parameter by at most about lr each, along its
+    # gradient's sign where that is not lost in rounding
+    step = net.get_params() - p
+    assert np.all(np.abs(step) <= 3.1e-3)
+    sure = np.abs(gr + 0.1 * p) > 0.2 * np.abs(gr + 0.1 * p).max()
+    assert np.all(step[sure] * (gr + 0.1 * p)[sure] < 0)
