@@ -118,7 +118,80 @@ FOT_DEV void load_loc(const uint16_t *__restrict__ p, uint32_t *loc) {
 }
 
 // ---- direct launches (atomics, global colour) -------------------------
-template <class F, bool SOA, bool ATOMIC, int LB = 1024>
+// The atomics loop's sums of one workgroup: a hash table in LDS, keyed by
+// point, in which the workgroup's increments are added before one FP64 atomic
+// per touched value goes to memory.  A point's home slot is its id modulo the
+// table's size, so points with neighbouring ids lie side by side and the flush
+// adds runs of consecutive values with consecutive lanes.
+//
+// The loop is bound by the atomic requests that leave the L2s, about 32 G/s
+// here, one per lane's row or value: one atomic per increment 359 us on the
+// GPS-ordered 1200x600 airfoil (SOA 267), whole rows by consecutive lanes but
+// unmerged 93, merged here 40 (SOA 40); shuffled 518 -> 206; mine 1024^2 on
+// compact blocks 559 -> 57, hex 64^3 255 -> 34.
+template <uint32_t TD> struct PointTable {
+  static constexpr uint32_t kBytesPerSlot = TD * 8 + 4;
+  // probes before an increment goes to memory by itself (a full table: a
+  // workgroup of a shuffled mesh touches as many points as it has slots)
+  static constexpr uint32_t kProbes = 8;
+  // as many slots as the workgroup's increments name points, at most: twice
+  // that measured slower on ordered meshes (46 us: more to clear and flush),
+  // half of it fills up (139 us)
+  static constexpr uint32_t slots_for(uint32_t n) {
+    uint32_t s = 64;
+    while (s < n) s *= 2;
+    return s;
+  }
+  uint32_t slots; // a power of two
+  double *vals;   // TD planes of `slots`
+  uint32_t *keys;
+  FOT_DEV PointTable(double *lds, uint32_t n) : slots(n), vals(lds) {
+    keys = reinterpret_cast<uint32_t *>(lds + size_t(n) * TD);
+  }
+  FOT_DEV void clear() {
+    for (uint32_t i = threadIdx.x; i < slots; i += blockDim.x) {
+      keys[i] = kExclusive;
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) vals[d * slots + i] = 0.0;
+    }
+  }
+  // the point's slot, or kExclusive when its first probes are all taken
+  FOT_DEV uint32_t find(uint32_t id) {
+    for (uint32_t k = 0; k < kProbes; ++k) {
+      const uint32_t i = (id + k) & (slots - 1);
+      const uint32_t was = atomicCAS(&keys[i], kExclusive, id);
+      if (was == kExclusive || was == id) return i;
+    }
+    return kExclusive;
+  }
+  template <bool SOA> FOT_DEV void add(double *out, uint32_t np, uint32_t id, const double *v) {
+    const uint32_t i = find(id);
+#pragma unroll
+    for (uint32_t d = 0; d < TD; ++d) {
+      if (i != kExclusive) unsafeAtomicAdd(&vals[d * slots + i], v[d]);
+      else atomic_add_f64(out + pidx<SOA>(np, id, TD, d), v[d]);
+    }
+  }
+  template <bool SOA> FOT_DEV void flush(double *out, uint32_t np) {
+    if constexpr (SOA) {
+      for (uint32_t i = threadIdx.x; i < slots; i += blockDim.x) {
+        const uint32_t id = keys[i];
+        if (id != kExclusive) {
+#pragma unroll
+          for (uint32_t d = 0; d < TD; ++d)
+            atomic_add_f64(out + size_t(d) * np + id, vals[d * slots + i]);
+        }
+      }
+    } else {
+      for (uint32_t j = threadIdx.x; j < slots * TD; j += blockDim.x) {
+        const uint32_t i = j / TD, d = j % TD, id = keys[i];
+        if (id != kExclusive) atomic_add_f64(out + size_t(id) * TD + d, vals[d * slots + i]);
+      }
+    }
+  }
+};
+
+template <class F, bool SOA, int LB = 1024>
 __global__ __launch_bounds__(LB) void eng_direct_kernel(EngineArgs a) {
   const uint32_t ind = blockIdx.x * blockDim.x + threadIdx.x;
   if (ind >= a.num_cells) return;
@@ -126,15 +199,42 @@ __global__ __launch_bounds__(LB) void eng_direct_kernel(EngineArgs a) {
   double inc[F::MD * F::TD];
   targets<F>(a, ind, tgt);
   F::template compute<SOA>(a, ind, tgt, inc);
-  add_increments<F, SOA, ATOMIC>(a.out, a.num_points[0], tgt, inc);
+  add_increments<F, SOA, false>(a.out, a.num_points[0], tgt, inc);
+}
+
+template <class F, bool SOA, int LB = 1024>
+__global__ __launch_bounds__(LB) void eng_atomic_kernel(EngineArgs a, uint32_t slots) {
+  extern __shared__ double lds[];
+  PointTable<F::TD> table(lds, slots);
+  table.clear();
+  const uint32_t ind = blockIdx.x * blockDim.x + threadIdx.x, np = a.num_points[0];
+  uint32_t tgt[F::MD];
+  double inc[F::MD * F::TD];
+  const bool live = ind < a.num_cells;
+  if (live) {
+    targets<F>(a, ind, tgt);
+    F::template compute<SOA>(a, ind, tgt, inc);
+  }
+  __syncthreads();
+  if (live) {
+#pragma unroll
+    for (uint32_t k = 0; k < F::MD; ++k)
+      table.template add<SOA>(a.out, np, tgt[k], inc + k * F::TD);
+  }
+  __syncthreads();
+  table.template flush<SOA>(a.out, np);
 }
 
 // res_calc over all edges with FP64 global atomics: the edge's two map rows
 // are 8-byte loads, consecutive lanes read consecutive rows (coalesced).
 template <bool SOA>
-__global__ __launch_bounds__(1024) void res_calc_atomic_kernel(EngineArgs a) {
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= a.num_cells) return;
+__global__ __launch_bounds__(1024) void res_calc_atomic_kernel(EngineArgs a, uint32_t slots) {
+  extern __shared__ double lds[];
+  PointTable<4> table(lds, slots);
+  table.clear();
+  const uint32_t ind = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool live = ind < a.num_cells;
+  const uint32_t e = live ? ind : a.num_cells - 1; // a valid edge for every lane
   const uint2 c = reinterpret_cast<const uint2 *>(a.maps[0])[e];
   const uint2 n = reinterpret_cast<const uint2 *>(a.maps[1])[e];
   const double *x = a.point_data[1], *q = a.point_data[2], *adt = a.point_data[3];
@@ -158,11 +258,13 @@ __global__ __launch_bounds__(1024) void res_calc_atomic_kernel(EngineArgs a) {
   double inc[8];
   res_calc_user(x1, x2, q1, q2, &adt1, &adt2, inc, inc + 4, 1, 1);
   const uint32_t np = a.num_points[0];
-#pragma unroll
-  for (uint32_t d = 0; d < 4; ++d) {
-    atomic_add_f64(a.out + pidx<SOA>(np, c.x, 4, d), inc[d]);
-    atomic_add_f64(a.out + pidx<SOA>(np, c.y, 4, d), inc[4 + d]);
+  __syncthreads();
+  if (live) {
+    table.add<SOA>(a.out, np, c.x, inc);
+    table.add<SOA>(a.out, np, c.y, inc + 4);
   }
+  __syncthreads();
+  table.flush<SOA>(a.out, np);
 }
 
 // ---- hierarchical launches --------------------------------------------
@@ -1978,6 +2080,21 @@ fot_status fot_loop::build_hierarchical() {
   return FOT_OK;
 }
 
+// Threads of an atomics workgroup.  Larger ones merge more increments of one
+// point before they reach memory: 1200x600 airfoil, GPS-ordered, 128 / 256 /
+// 512 / 1024 threads 59 / 94 / 40 / 42 us (256 fill their table, the next
+// power of two, to the brim).  Meshes too small to fill the chip that way run
+// 128, by their increments (edges of two cells, 9 000 to 90 000: 3.7-5.0 us
+// against 4.3-5.1 with 512; 160 000: 8.6 against 6.7; lulesh 48^3, 110 000
+// elements of eight nodes: 31 against 21), mini_aero's registers ask for 256
+// (48^3: 34 us against 42), and the table has to fit the LDS.
+template <class F> uint32_t atomic_threads(uint32_t cells) {
+  uint32_t n = uint64_t(F::MD) * cells < (1u << 18) ? 128u : kSmallBound<F> < 1024 ? 256u : 512u;
+  while (PointTable<F::TD>::slots_for(F::MD * n) * PointTable<F::TD>::kBytesPerSlot > 144u * 1024u)
+    n /= 2;
+  return n;
+}
+
 fot_status fot_loop::enqueue(hipStream_t s) {
   if (desc.num_cells == 0) return FOT_OK; // nothing to launch
   const fot_status st = dispatch(&f, desc.soa, [&]<class F, bool SOA>() -> fot_status {
@@ -1986,16 +2103,18 @@ fot_status fot_loop::enqueue(hipStream_t s) {
     constexpr int LB = kSmallBound<F>;
     const uint32_t dbs = std::min<uint32_t>(bs, LB);
     if (cfg.strategy == FOT_STRATEGY_ATOMIC) {
+      const uint32_t at = atomic_threads<F>(desc.num_cells);
+      const uint32_t slots = PointTable<F::TD>::slots_for(F::MD * at);
+      const uint32_t lds = slots * PointTable<F::TD>::kBytesPerSlot;
+      const dim3 grid((desc.num_cells + at - 1) / at);
       if constexpr (std::is_same<F, ResCalcF>::value)
-        hipLaunchKernelGGL((res_calc_atomic_kernel<SOA>), dim3((desc.num_cells + bs - 1) / bs),
-                           dim3(bs), 0, s, base);
+        hipLaunchKernelGGL((res_calc_atomic_kernel<SOA>), grid, dim3(at), lds, s, base, slots);
       else
-        hipLaunchKernelGGL((eng_direct_kernel<F, SOA, true, LB>),
-                           dim3((desc.num_cells + dbs - 1) / dbs), dim3(dbs), 0, s, base);
+        hipLaunchKernelGGL((eng_atomic_kernel<F, SOA, LB>), grid, dim3(at), lds, s, base, slots);
     } else if (cfg.strategy == FOT_STRATEGY_GLOBAL_COLOUR) {
       for (const EngineArgs &a : colour_args) {
         if (a.num_cells == 0) continue;
-        hipLaunchKernelGGL((eng_direct_kernel<F, SOA, false, LB>),
+        hipLaunchKernelGGL((eng_direct_kernel<F, SOA, LB>),
                            dim3((a.num_cells + dbs - 1) / dbs), dim3(dbs), 0, s, a);
       }
     } else if (owner) {

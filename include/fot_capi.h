@@ -480,7 +480,8 @@ typedef struct {
 
 typedef struct {
   uint32_t strategy;      /* fot_strategy */
-  uint32_t block_size;    /* threads (atomic/global) or cells per block */
+  uint32_t block_size;    /* threads (global colour) or cells per block; the
+                             atomics loop sizes its own workgroups */
   const uint32_t *partition; /* HOST, nullable: block id per cell */
   uint32_t use_graph;     /* capture one iteration in a hipGraph */
   uint32_t flags;         /* FOT_LOOP_* */

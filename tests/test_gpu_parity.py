@@ -225,6 +225,25 @@ def test_res_calc_atomic_run_to_run(gpu):
     assert_close_scaled(a.point_data[0], b.point_data[0], S, what="atomic run to run")
 
 
+@pytest.mark.parametrize("P,soa", [(1, False), (4, False), (4, True), (8, True)])
+@pytest.mark.parametrize("edges", ["one short", "shuffled", "ordered", "star"])
+def test_atomic_point_table(gpu, P, soa, edges):
+    """The atomics loop's per-workgroup point table around the size where the
+    workgroups change (2^18 increments), on a shuffled mesh (more points than the
+    table has free slots), an ordered one, and with every edge on one point."""
+    p = mine_problem(N=260, M=254, P=P, C=P, soa=soa, shuffle=edges != "ordered")
+    assert p.num_cells > 1 << 17
+    if edges == "one short":
+        p.maps = [p.maps[0][:(1 << 17) - 1]]
+        p.cell_data = [p.cell_data[0][:, :(1 << 17) - 1].copy()]
+    if edges == "star":
+        p.maps[0][:, 0] = 5
+        p.maps[0][p.maps[0][:, 1] == 5, 1] = 6
+    ref, S = _serial(p, O.MINE2, 1)
+    p.gpu_loop(capi.functor(capi.KERNEL_MINE, 2, P, P), capi.STRATEGY_ATOMIC, 1)
+    assert_close_scaled(p.point_data[0], ref, S, what="mine atomic")
+
+
 @pytest.mark.parametrize("P,C,soa", [(4, 4, False), (4, 1, True), (1, 1, False), (8, 8, True)])
 def test_mine_strategies(gpu, P, C, soa):
     f = capi.functor(capi.KERNEL_MINE, 2, P, C)
