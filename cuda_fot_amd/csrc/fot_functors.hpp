@@ -571,18 +571,19 @@ struct GetaccF {
 
 // The point data a functor reads through its cells' mapping-0 ids (`tgt` in
 // compute), which a hierarchical block can stage in LDS with its cache:
-// slot (-1: none) and values per point.
+// slot (-1: none) and values per point; cell_dim: the values of cell data 0
+// of the functors that eng_gather_kernel stages.
 template <class F> struct StagedInput {
   static constexpr int slot = -1;
   static constexpr uint32_t dim = 0;
 };
 template <> struct StagedInput<MiniAeroF> { // the 28 cell values
   static constexpr int slot = 1;
-  static constexpr uint32_t dim = 28;
+  static constexpr uint32_t dim = 28, cell_dim = 12;
 };
 template <> struct StagedInput<LuleshF> { // node coordinates
   static constexpr int slot = 1;
-  static constexpr uint32_t dim = 3;
+  static constexpr uint32_t dim = 3, cell_dim = 3;
 };
 template <> struct StagedInput<VolnaF> { // cell volumes
   static constexpr int slot = 1;
@@ -605,6 +606,28 @@ template <int SLOT> struct LdsArgs {
   FOT_DEV uint32_t ps(uint32_t k) const { return k == uint32_t(SLOT) ? m : a.ps(k); }
   FOT_DEV const double *cd(uint32_t k) const { return a.cd(k); }
   FOT_DEV uint32_t cs() const { return a.cs(); }
+};
+
+// Staged input as rows of a constant, odd number of values per point: a
+// point's values sit at immediate offsets (two to an LDS read), and rows
+// start in different banks.
+template <class F> struct StagedRows {
+  static constexpr uint32_t row = StagedInput<F>::dim | 1u;
+};
+
+// The engine arguments seen by a functor's SOA form whose staged input is in
+// LDS rows and whose cell data 0 is in registers: `tgt` holds block-local ids
+// times the row, a point's values are one apart, and so are the cell's; other
+// cell data is the caller's at the cell's position (`ind` is 0).
+template <int SLOT> struct LdsRows {
+  const EngineArgs &a;
+  const double *staged, *cell;
+  uint32_t pos;
+  static constexpr bool kStreamCells = false;
+  FOT_DEV const double *pd(uint32_t k) const { return k == uint32_t(SLOT) ? staged : a.pd(k); }
+  FOT_DEV uint32_t ps(uint32_t k) const { return k == uint32_t(SLOT) ? 1u : a.ps(k); }
+  FOT_DEV const double *cd(uint32_t k) const { return k == 0 ? cell : a.cd(k) + pos; }
+  FOT_DEV uint32_t cs() const { return 1u; }
 };
 
 // Mapping-0 ids of cell `ind` (AOS row).

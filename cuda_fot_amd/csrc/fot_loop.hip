@@ -25,6 +25,8 @@ constexpr uint32_t kNumXcd = 8; // MI355X: 8 XCDs of 32 CUs
 // MI355X's Infinity Cache (MALL): the memory-side cache in front of HBM
 constexpr uint64_t kInfinityCacheBytes = uint64_t(256) << 20;
 typedef double dvec2 __attribute__((ext_vector_type(2)));
+// a pair of values of a caller's array, which only has to be 8-byte aligned
+typedef double dvec2u __attribute__((ext_vector_type(2), aligned(8)));
 
 // Workgroups are dispatched round-robin over the XCDs; this bijection gives
 // each XCD a contiguous run of plan blocks, so neighbouring blocks (which
@@ -48,6 +50,12 @@ struct HierDev {
   // when no other block touches the point; partial sums [slot][TD]
   const uint32_t *wslot;
   double *partial;
+  // gather accumulation (eng_gather_kernel): block records (first cell, cells,
+  // first cached entry, cached points) and per cached entry the increments it
+  // adds, in order, as 4 or 8 (`wide`) 16-bit places in the block's LDS planes
+  const uint4 *rec;
+  const uint32_t *lists;
+  uint32_t wide;
 };
 
 constexpr uint32_t kExclusive = 0xffffffffu;
@@ -443,6 +451,207 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_h
     }
   }
   publish<DEP>(dd, b, gen);
+}
+
+// ---- gather accumulation ----------------------------------------------------
+// The hierarchical kernel whose points gather: every cell stores its
+// increments in LDS planes and every cached point adds the ones it is due, from
+// a list in the plan, in thread-colour order (then by the cell's slots): the
+// additions of eng_hier_kernel in its order, the same bits, but independent
+// over the points, where the colour loop runs a chain of dependent LDS
+// read-add-writes and a barrier per colour.  The lists take the place of the
+// local ids and colours, and come with the points' ids and slots at the
+// block's start, so the sums go out without another round trip.
+//
+// What bounds a block is its chain of round trips (record, ids, values, the
+// output to add to) against the blocks a CU holds; past that, the bytes.  Two-
+// phase, colour loop / this kernel, per launch: hex 103x110x97, blocks of 512,
+// 70 / 58 us (5.2 TB/s); hex 64^3 as a step 29 / 20; getacc 1024^2 58 / 52;
+// mine 1024^2 36 / 35 (already at 5.5 TB/s).
+//
+// Increments are handled kPassDims values per pass, so that the planes of a
+// 512-thread block take 32 KB.  Plans with a point of more than 8 increments
+// in a block, or with more than two points per thread, keep the colour loop.
+template <class F>
+constexpr uint32_t kPassDims = F::MD == 2 && F::TD <= 5 ? F::TD : F::MD >= 8 ? 1 : 8 / F::MD;
+// The functors whose gathered input is staged in LDS: mini_aero's 28 values a
+// cell (a lane per row took 64 cache lines per load and kept the L1 at 0.75
+// accesses a cycle: 113 us per launch at 80^3, blocks of 128; staged row by
+// row by 16 lanes 90) and lulesh's coordinates (96^3, blocks of 512: 52
+// against 41).  Staging by a lane per row or value, or issued after the cell's
+// own values, measured no faster than gathering.
+template <class F>
+constexpr bool kStagesInput = std::is_same_v<F, fot::MiniAeroF> || std::is_same_v<F, fot::LuleshF>;
+// the functors that read point data by their cells' mapping-0 ids
+template <class F>
+constexpr bool kNeedsTargets = !std::is_same_v<F, HexScatterF> && !std::is_same_v<F, GetaccF>;
+
+// LDS of a block of `threads` threads and m cached points
+template <class F> constexpr uint32_t gather_lds(uint32_t threads, uint32_t m) {
+  const uint32_t planes = 8u * std::min(kPassDims<F>, F::TD) * (F::MD * threads + 1);
+  const uint32_t staged = kStagesInput<F> ? 8u * StagedRows<F>::row * m : 0u;
+  return std::max(planes, staged);
+}
+
+// Staging of points with wide rows (AOS): 16 lanes take the consecutive pairs
+// of a point's row, and a thread has kRows rows in flight (14: 112 rows of a
+// 128-thread block, more than nearly all of them cache; with 10 half the
+// blocks paid a second pair of round trips, 101 against 90 us per launch at
+// 80^3 together with the next line's).  load() comes first of a block's loads
+// and stage() waits for the ids alone, not for the cell's values from HBM.
+template <class F, bool SOA> struct RowIds {
+  static constexpr bool kUsed = kStagesInput<F> && !SOA && StagedInput<F>::dim >= 8;
+  static constexpr uint32_t kRows = kUsed ? 14 : 1, kPairs = kUsed ? StagedInput<F>::dim / 2 : 1;
+  static_assert(kPairs <= 16 && (!kUsed || StagedInput<F>::dim % 2 == 0));
+  uint32_t id[kRows];
+  FOT_DEV void load(const uint32_t *cached, uint32_t m) {
+    if constexpr (kUsed) {
+#pragma unroll
+      for (uint32_t q = 0; q < kRows; ++q)
+        id[q] = cached[min((threadIdx.x + q * blockDim.x) / 16, m - 1)];
+    }
+  }
+  FOT_DEV void stage(const double *src, double *lds, uint32_t m) const {
+    constexpr uint32_t dim = StagedInput<F>::dim, row = StagedRows<F>::row;
+    const uint32_t pair = min(threadIdx.x % 16, kPairs - 1);
+    dvec2u in[kRows];
+#pragma unroll
+    for (uint32_t q = 0; q < kRows; ++q)
+      in[q] = *reinterpret_cast<const dvec2u *>(src + size_t(id[q]) * dim + 2 * pair);
+    // one wait for all of them (see res_calc_owner2_kernel)
+#pragma unroll
+    for (uint32_t q = 0; q < kRows; ++q) asm volatile("" ::"v"(in[q].x), "v"(in[q].y));
+#pragma unroll
+    for (uint32_t q = 0; q < kRows; ++q) {
+      const uint32_t i = (threadIdx.x + q * blockDim.x) / 16;
+      if (i < m && threadIdx.x % 16 < kPairs)
+        lds[i * row + 2 * pair] = in[q].x, lds[i * row + 2 * pair + 1] = in[q].y;
+    }
+  }
+};
+
+// R: rounds of points a thread takes (at most R * blockDim.x cached points).
+// Without write slots (one launch per block colour) every point is added in
+// place.
+template <class F, bool SOA, int R, int LB = 1024, bool NTC = false>
+__global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_gather_kernel(
+    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, uint32_t blk_begin,
+    uint32_t nbc) {
+  constexpr uint32_t MD = F::MD, TD = F::TD, PD = std::min(kPassDims<F>, TD);
+  extern __shared__ double lds[];
+  const uint4 rec = h.rec[blk_begin + xcd_block(blockIdx.x, nbc)];
+  const uint32_t tid = threadIdx.x, T = blockDim.x, e0 = rec.x, ne = rec.y, c0 = rec.z, m = rec.w;
+  // the points' lists, ids and slots are in flight with the cell's values
+  // (a wide staged row's ids first: its values wait for them)
+  RowIds<F, SOA> rows;
+  rows.load(h.cached + c0, m);
+  uint4 list[R];
+  uint32_t g[R], slot[R];
+  {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t entry = c0 + min(tid + r * T, m - 1);
+      if (h.wide) {
+        list[r] = reinterpret_cast<const uint4 *>(h.lists)[entry];
+      } else {
+        const uint2 w = reinterpret_cast<const uint2 *>(h.lists)[entry];
+        list[r] = make_uint4(w.x, w.y, 0u, 0u);
+      }
+      g[r] = h.cached[entry];
+      slot[r] = h.wslot ? h.wslot[entry] : kExclusive;
+    }
+  }
+  const uint32_t pos = e0 + min(tid, ne - 1);
+  uint32_t tgt[MD];
+  double inc[MD * TD];
+  if constexpr (kStagesInput<F>) {
+    using SI = StagedInput<F>;
+    load_loc<MD>(h.loc + size_t(pos) * MD, tgt);
+    // (the cell's own values come while the points are staged)
+    double cell[SI::cell_dim];
+#pragma unroll
+    for (uint32_t k = 0; k < SI::cell_dim; ++k)
+      cell[k] = load_once<NTC>(&a.cd(0)[pos + size_t(k) * a.cs()]);
+    const double *src = a.pd(SI::slot);
+    const uint32_t n = a.ps(SI::slot);
+    constexpr uint32_t row = StagedRows<F>::row;
+    if constexpr (SOA || SI::dim < 8) {
+      double in[R][SI::dim];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (uint32_t k = 0; k < SI::dim; ++k) in[r][k] = src[pidx<SOA>(n, g[r], SI::dim, k)];
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (tid + r * T < m) {
+#pragma unroll
+          for (uint32_t k = 0; k < SI::dim; ++k) lds[(tid + r * T) * row + k] = in[r][k];
+        }
+    } else {
+      rows.stage(src, lds, m);
+      for (uint32_t i0 = rows.kRows * (T / 16); i0 < m; i0 += rows.kRows * (T / 16)) {
+        rows.load(h.cached + c0 + i0, m - i0);
+        rows.stage(src, lds + size_t(i0) * row, m - i0);
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < MD; ++k) tgt[k] *= row;
+    __syncthreads();
+    if (tid < ne) F::template compute<true>(LdsRows<SI::slot>{a, lds, cell, pos}, 0, tgt, inc);
+    __syncthreads(); // the planes take the staged values' place
+  } else {
+    if constexpr (kNeedsTargets<F>) targets<F>(a, pos, tgt);
+    if (tid < ne) F::template compute<SOA>(a, pos, tgt, inc);
+  }
+  const uint32_t np = a.num_points[0], stride = MD * T + 1; // + a zero for empty places
+  double v[R][TD];
+#pragma unroll
+  for (uint32_t d0 = 0; d0 < TD; d0 += PD) {
+    if (d0) __syncthreads();
+    if (tid < ne) {
+#pragma unroll
+      for (uint32_t p = 0; p < PD; ++p)
+        if (d0 + p < TD) {
+#pragma unroll
+          for (uint32_t k = 0; k < MD; ++k)
+            lds[p * stride + k * T + tid] = inc[k * TD + d0 + p];
+        }
+    }
+    if (d0 == 0 && tid < PD) lds[tid * stride + MD * T] = 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t at[8] = {list[r].x & 0xffffu, list[r].x >> 16, list[r].y & 0xffffu,
+                              list[r].y >> 16,     list[r].z & 0xffffu, list[r].z >> 16,
+                              list[r].w & 0xffffu, list[r].w >> 16};
+#pragma unroll
+      for (uint32_t p = 0; p < PD; ++p) {
+        if (d0 + p >= TD) continue;
+        double s = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) s += lds[p * stride + at[j]];
+        if (h.wide) {
+#pragma unroll
+          for (uint32_t j = 4; j < 8; ++j) s += lds[p * stride + at[j]];
+        }
+        v[r][d0 + p] = s;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (tid + r * T >= m) continue;
+    if (slot[r] == kExclusive) {
+      double o[TD];
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) o[d] = a.out[pidx<SOA>(np, g[r], TD, d)];
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) a.out[pidx<SOA>(np, g[r], TD, d)] = o[d] + v[r][d];
+    } else {
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) h.partial[size_t(slot[r]) * TD + d] = v[r][d];
+    }
+  }
 }
 
 // res_calc hierarchical with the block's cells' q and adt staged in LDS next
@@ -1361,6 +1570,33 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
                      lds, s, a, h, dd, b0, nbc);
 }
 
+// Launches eng_gather_kernel<F, SOA, R>.
+template <class F, bool SOA, int R>
+void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
+                   const EngineArgs &a, const HierDev &h, uint32_t b0, uint32_t nbc,
+                   bool stream_cells) {
+  constexpr int SB = kSmallBound<F>;
+  const bool small = threads <= uint32_t(SB);
+  if constexpr (kStreamsCells<F>) {
+    if (stream_cells) {
+      const StreamCellArgs sa{a};
+      if (small)
+        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB, true>), dim3(grid), dim3(threads),
+                           lds, s, sa, h, b0, nbc);
+      else
+        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, 1024, true>), dim3(grid), dim3(threads),
+                           lds, s, sa, h, b0, nbc);
+      return;
+    }
+  }
+  if (small)
+    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB>), dim3(grid), dim3(threads), lds, s, a, h,
+                       b0, nbc);
+  else
+    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R>), dim3(grid), dim3(threads), lds, s, a, h,
+                       b0, nbc);
+}
+
 // Values per point of a functor's staged input (0: none).
 uint32_t staged_input_dim(const fot_functor &f) {
   uint32_t d = 0;
@@ -1395,6 +1631,8 @@ struct fot_loop {
   std::vector<uint32_t> colour_blk_off;
   uint32_t lds_bytes = 0, threads = 0;
   bool staged = false;
+  uint32_t gather_rounds = 1;
+  bool gather = false;   // hierarchical: points gather their increments (eng_gather_kernel)
   bool stage_pd = false; // generic hierarchical: the functor's staged input in LDS
   bool dep_order = false;
   bool owner = false;
@@ -1521,6 +1759,11 @@ struct fot_loop {
     return FOT_OK;
   }
 
+  // the plan of eng_gather_kernel, when the blocks allow it: sets `gather`
+  fot_status build_gather(const std::vector<uint32_t> &blk_cell_off,
+                          const std::vector<uint32_t> &blk_cache_off,
+                          const std::vector<uint16_t> &loc,
+                          const std::vector<uint32_t> &plan_cell);
   fot_status build_atomic();
   fot_status build_global_colour();
   fot_status build_hierarchical();
@@ -1608,6 +1851,117 @@ static void sort_positions_by_local_ids(const std::vector<uint32_t> &blk_cell_of
   }
 }
 
+// Blocks by where their cells lie in the mesh as given: by partition id, then
+// by their lowest cell.  The plan's order is by block colour, which keeps any
+// two blocks that share a point apart; a two-phase launch takes its blocks in
+// any order, and in this one blocks that share points run side by side on one
+// XCD and find them in its L2.
+static std::vector<uint32_t> mesh_order(const std::vector<uint32_t> &blk_cell_off,
+                                        const std::vector<uint32_t> &cells,
+                                        const uint32_t *partition) {
+  const uint32_t nb = uint32_t(blk_cell_off.size()) - 1;
+  std::vector<uint64_t> key(nb);
+  for (uint32_t b = 0; b < nb; ++b) {
+    const uint32_t low = *std::min_element(cells.begin() + blk_cell_off[b],
+                                           cells.begin() + blk_cell_off[b + 1]);
+    key[b] = (uint64_t(partition ? partition[low] : 0u) << 32) | low;
+  }
+  std::vector<uint32_t> order(nb);
+  std::iota(order.begin(), order.end(), 0u);
+  std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t c) { return key[a] < key[c]; });
+  return order;
+}
+// The blocks' runs of v (off[b] * each to off[b + 1] * each) in another order
+template <class T>
+static void permute_runs(const std::vector<uint32_t> &order, const std::vector<uint32_t> &off,
+                         std::vector<T> &v, uint32_t each) {
+  std::vector<T> out;
+  out.reserve(v.size());
+  for (uint32_t b : order)
+    out.insert(out.end(), v.begin() + size_t(off[b]) * each, v.begin() + size_t(off[b + 1]) * each);
+  v.swap(out);
+}
+// ... and, as the last array on these offsets, the offsets with it
+template <class T>
+static void permute_offsets(const std::vector<uint32_t> &order, std::vector<uint32_t> &off,
+                            std::vector<T> &v, uint32_t each) {
+  permute_runs(order, off, v, each);
+  std::vector<uint32_t> out{0};
+  for (uint32_t b : order) out.push_back(out.back() + off[b + 1] - off[b]);
+  off.swap(out);
+}
+
+fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
+                                  const std::vector<uint32_t> &blk_cache_off,
+                                  const std::vector<uint16_t> &loc,
+                                  const std::vector<uint32_t> &plan_cell) {
+  const uint32_t md = desc.mesh_dim[0], nb = uint32_t(blk_cell_off.size()) - 1;
+  uint32_t lds = 0;
+  bool targets = false, stages = false;
+  fot_status st = dispatch(&f, desc.soa, [&]<class F, bool SOA>() -> fot_status {
+    for (uint32_t b = 0; b < nb; ++b)
+      lds = std::max(lds, gather_lds<F>(threads, blk_cache_off[b + 1] - blk_cache_off[b]));
+    stages = kStagesInput<F>;
+    targets = kNeedsTargets<F> && !stages;
+    return FOT_OK;
+  });
+  if (st != FOT_OK) return st;
+  if (stage_pd && !stages) return FOT_OK; // eng_hier_kernel stages the others' input
+  if (lds > 160u * 1024u || md * threads > 0xfffeu) return FOT_OK;
+  // A point's increments in the order of the plan's cells, which are sorted by
+  // thread colour, then by the cell's slots.
+  const uint16_t none = uint16_t(md * threads);
+  std::vector<uint16_t> lists(size_t(blk_cache_off[nb]) * 8, none);
+  std::vector<uint8_t> count;
+  std::vector<uint4> rec(nb);
+  uint32_t longest = 0, most = 0;
+  for (uint32_t b = 0; b < nb; ++b) {
+    const uint32_t e0 = blk_cell_off[b], ne = blk_cell_off[b + 1] - e0;
+    const uint32_t c0 = blk_cache_off[b], m = blk_cache_off[b + 1] - c0;
+    rec[b] = make_uint4(e0, ne, c0, m);
+    most = std::max(most, m);
+    count.assign(m, 0);
+    for (uint32_t i = 0; i < ne; ++i)
+      for (uint32_t k = 0; k < md; ++k) {
+        const uint32_t l = loc[size_t(e0 + i) * md + k];
+        if (count[l] == 8) return FOT_OK;
+        lists[size_t(c0 + l) * 8 + count[l]++] = uint16_t(k * threads + i);
+        longest = std::max<uint32_t>(longest, count[l]);
+      }
+  }
+  if (most > 2 * threads) return FOT_OK;
+  gather_rounds = most > threads ? 2 : 1;
+  if (longest <= 4) {
+    const size_t n = lists.size() / 8;
+    for (size_t i = 0; i < n; ++i)
+      for (size_t j = 0; j < 4; ++j) lists[4 * i + j] = lists[8 * i + j];
+    lists.resize(4 * n);
+  }
+  uint4 *d4 = nullptr;
+  uint16_t *d16 = nullptr;
+  uint32_t *d32 = nullptr;
+  if ((st = upload(rec.data(), rec.size(), &d4)) != FOT_OK) return st;
+  hier.rec = d4;
+  if ((st = upload(lists.data(), lists.size(), &d16)) != FOT_OK) return st;
+  hier.lists = reinterpret_cast<const uint32_t *>(d16);
+  hier.wide = longest > 4;
+  if (targets) {
+    std::vector<uint32_t> ids(plan_cell.size() * md);
+    for (size_t i = 0; i < plan_cell.size(); ++i)
+      std::memcpy(&ids[i * md], desc.cell_to_node[0] + size_t(plan_cell[i]) * md,
+                  md * sizeof(uint32_t));
+    if ((st = upload(ids.data(), ids.size(), &d32)) != FOT_OK) return st;
+    plan_args.maps[0] = d32;
+  }
+  if (stages) {
+    if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
+    hier.loc = d16;
+  }
+  lds_bytes = lds;
+  gather = true;
+  return FOT_OK;
+}
+
 fot_status fot_loop::build_hierarchical() {
   fot_status st;
   const uint32_t md = desc.mesh_dim[0];
@@ -1683,6 +2037,9 @@ fot_status fot_loop::build_hierarchical() {
                               cfg.block_size, plan);
   if (st != FOT_OK) return st;
   num_plan_colours = uint32_t(plan.colours.size());
+  loc.reserve(size_t(desc.num_cells) * md);
+  colour.reserve(desc.num_cells);
+  plan_cell.reserve(desc.num_cells);
   for (const HostColour &hc : plan.colours) {
     const uint32_t nb = uint32_t(hc.num_cell_colours.size());
     const uint32_t n = uint32_t(hc.cell_colours.size());
@@ -1715,6 +2072,25 @@ fot_status fot_loop::build_hierarchical() {
   }
   }
   const uint32_t nb_total = colour_blk_off.back();
+  // block order of a two-phase launch: launch_of[plan block], the plan's blocks
+  // being in colour order
+  std::vector<uint32_t> launch_of;
+  if (two_phase) {
+    const std::vector<uint32_t> order =
+        mesh_order(blk_cell_off, plan_cell, cfg.partition);
+    launch_of.resize(nb_total);
+    for (uint32_t j = 0; j < nb_total; ++j) launch_of[order[j]] = j;
+    permute_runs(order, blk_cell_off, plan_cell, 1);
+    permute_runs(order, blk_cell_off, colour, 1);
+    for (uint32_t m = 1; m < desc.num_mappings; ++m)
+      if (!plan_maps[m].empty())
+        permute_runs(order, blk_cell_off, plan_maps[m], desc.mesh_dim[m]);
+    permute_offsets(order, blk_cell_off, loc, md);
+    permute_offsets(order, blk_cache_off, cached, 1);
+    std::vector<uint8_t> ncol(nb_total);
+    for (uint32_t j = 0; j < nb_total; ++j) ncol[j] = blk_ncol[order[j]];
+    blk_ncol.swap(ncol);
+  }
   uint32_t *d32 = nullptr;
   uint16_t *d16 = nullptr;
   uint8_t *d8 = nullptr;
@@ -1729,12 +2105,6 @@ fot_status fot_loop::build_hierarchical() {
   if (owner_rc) cached.resize(cached.size() + kOwnerPad, 0u);
   if ((st = upload(cached.data(), cached.size(), &d32)) != FOT_OK) return st;
   hier.cached = d32;
-  if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
-  hier.loc = d16;
-  if ((st = upload(colour.data(), colour.size(), &d8)) != FOT_OK) return st;
-  hier.colour = d8;
-  if ((st = upload(blk_ncol.data(), blk_ncol.size(), &d8)) != FOT_OK) return st;
-  hier.blk_ncol = d8;
   if (owner) {
     if ((st = upload(blk_owned.data(), blk_owned.size(), &d32)) != FOT_OK) return st;
     hier.blk_owned = d32;
@@ -1869,12 +2239,12 @@ fot_status fot_loop::build_hierarchical() {
     if ((st = upload(plan_maps[m].data(), plan_maps[m].size(), &d32)) != FOT_OK) return st;
     plan_args.maps[m] = d32;
   }
-  if ((st = gather_cell_data(plan_cell.data(), uint32_t(plan_cell.size()), plan_args)) != FOT_OK) return st;
+  if ((st = gather_cell_data(plan_cell.data(), uint32_t(plan_cell.size()), plan_args)) != FOT_OK)
+    return st;
   if (two_phase) {
-    // Blocks in plan (colour-major) order; a point's partial slots are
-    // handed out in that order, so ascending slots are ascending block
-    // colours.  Slots of one block are consecutive (its shared points in
-    // cache order): its partial stores are contiguous.
+    // Slots of one block are consecutive (its shared points in cache order),
+    // so its partial stores are contiguous; a point's list names them in the
+    // plan's order, which is by block colour.
     std::vector<uint32_t> touch(desc.num_points[0], 0);
     for (uint32_t i = 0; i < blk_cache_off[nb_total]; ++i) ++touch[cached[i]];
     std::vector<uint32_t> rank(desc.num_points[0], 0xffffffffu), pt, off{0};
@@ -1886,15 +2256,14 @@ fot_status fot_loop::build_hierarchical() {
       }
     std::vector<uint32_t> wslot(blk_cache_off[nb_total]), slots(off.back()), fill(pt.size(), 0);
     uint32_t next = 0;
-    for (uint32_t i = 0; i < blk_cache_off[nb_total]; ++i) {
-      const uint32_t r = rank[cached[i]];
-      if (r == 0xffffffffu) {
-        wslot[i] = kExclusive;
-      } else {
-        wslot[i] = next;
-        slots[off[r] + fill[r]++] = next++;
-      }
-    }
+    for (uint32_t i = 0; i < blk_cache_off[nb_total]; ++i)
+      wslot[i] = rank[cached[i]] == 0xffffffffu ? kExclusive : next++;
+    for (uint32_t j : launch_of)
+      for (uint32_t i = blk_cache_off[j]; i < blk_cache_off[j + 1]; ++i)
+        if (wslot[i] != kExclusive) {
+          const uint32_t r = rank[cached[i]];
+          slots[off[r] + fill[r]++] = wslot[i];
+        }
     merge_n = uint32_t(pt.size());
     if ((st = upload(wslot.data(), wslot.size(), &d32)) != FOT_OK) return st;
     hier.wslot = d32;
@@ -1992,6 +2361,17 @@ fot_status fot_loop::build_hierarchical() {
   ept = (owner && f.kernel == FOT_KERNEL_RES_CALC && (cfg.flags & FOT_LOOP_TWO_PER_THREAD)) ? 2 : 1;
   threads = std::max<uint32_t>(64, ((max_block + ept - 1) / ept + 63) / 64 * 64);
   if (threads > 1024) return fail(FOT_ERR_UNSUPPORTED, "blocks above 1024 cells");
+  if (!owner && !dep_order && !staged &&
+      (st = build_gather(blk_cell_off, blk_cache_off, loc, plan_cell)) != FOT_OK)
+    return st;
+  if (!gather) {
+    if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
+    hier.loc = d16;
+    if ((st = upload(colour.data(), colour.size(), &d8)) != FOT_OK) return st;
+    hier.colour = d8;
+    if ((st = upload(blk_ncol.data(), blk_ncol.size(), &d8)) != FOT_OK) return st;
+    hier.blk_ncol = d8;
+  }
   if (owner && f.kernel == FOT_KERNEL_RES_CALC) {
     // the staging rounds cover max(cached, nodes) of every block
     uint32_t most = max_nodes;
@@ -2194,7 +2574,12 @@ fot_status fot_loop::enqueue(hipStream_t s) {
           done = true;
         }
       }
-      if (!done)
+      if (gather) {
+        if (gather_rounds == 1)
+          launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, 0u, nb, nontemporal);
+        else
+          launch_gather<F, SOA, 2>(nb, threads, lds_bytes, s, plan_args, hier, 0u, nb, nontemporal);
+      } else if (!done)
         launch_eng_hier<F, SOA, 2>(stage_pd, nb, threads, lds_bytes, s, plan_args, hier, dep,
                                    0u, nb, nontemporal);
       if (merge_n)
@@ -2212,7 +2597,12 @@ fot_status fot_loop::enqueue(hipStream_t s) {
             continue;
           }
         }
-        launch_eng_hier<F, SOA, 0>(stage_pd, nbc, threads, lds_bytes, s, plan_args, hier, dep,
+        if (gather && gather_rounds == 1)
+          launch_gather<F, SOA, 1>(nbc, threads, lds_bytes, s, plan_args, hier, b0, nbc, false);
+        else if (gather)
+          launch_gather<F, SOA, 2>(nbc, threads, lds_bytes, s, plan_args, hier, b0, nbc, false);
+        else
+          launch_eng_hier<F, SOA, 0>(stage_pd, nbc, threads, lds_bytes, s, plan_args, hier, dep,
                                    b0, nbc);
       }
     }

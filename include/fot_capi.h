@@ -491,7 +491,8 @@ typedef struct {
  * q and adt; mini_aero: the cell values; lulesh: the node coordinates;
  * volna: the cell volumes; mine: the iterate).  Functors other than res_calc
  * gather per cell as without the flag when the staged values and the cache
- * do not fit in LDS together. */
+ * do not fit in LDS together.  mini_aero and lulesh are staged without the
+ * flag too where that is faster. */
 #define FOT_LOOP_STAGE_INPUTS 1u
 /* hierarchical: single launch, blocks ordered by per-block dependency
  * flags instead of one launch per block colour */

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from cuda_fot_amd import capi, plan
+from cuda_fot_amd import Problem, capi, meshgen, plan
 from helpers import (airfoil_problem, assert_bitwise, assert_close_scaled, hex_problem,
                      mine_problem, oracle_of)
 
@@ -265,6 +265,47 @@ def test_mine_strategies(gpu, P, C, soa):
     a = mine_problem(P=P, C=C, soa=soa)
     a.gpu_loop(f, capi.STRATEGY_ATOMIC, ITERS)
     assert_close_scaled(a.point_data[0], ref_serial, S, what="mine atomic")
+
+
+def _gather_mesh(kind):
+    """Cells of 2 or 8 points around the limits of the gathered sums: lists of
+    exactly 4, 8 and 9 increments per point in a block, one and two points per
+    thread and one more, cells naming a point twice, ragged blocks."""
+    rng = np.random.default_rng(7)
+    if kind.startswith("hubs"):  # points of that many edges each
+        d = int(kind[4:])
+        hubs = np.repeat(np.arange(60), d)
+        maps = np.stack([hubs, 60 + np.arange(hubs.size)], 1)
+        return maps[rng.permutation(hubs.size)], 60 + hubs.size, 2, 64
+    if kind == "twice":
+        maps = np.stack([np.arange(500) % 97, np.arange(500) * 7 % 97], 1)
+        maps[::9, 1] = maps[::9, 0]
+        return maps, 97, 2, 128
+    cells, bs = {"two": (16 * 9 + 3, 16), "three": (17 * 9, 17), "one": (64, 8)}[kind]
+    return rng.permutation(cells * 8).reshape(cells, 8), cells * 8, 8, bs
+
+
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("kind", ["hubs4", "hubs8", "hubs9", "twice", "one", "two", "three"])
+def test_gathered_sums_at_their_limits(gpu, kind, soa):
+    maps, n, md, bs = _gather_mesh(kind)
+    k = {2: O.MINE2, 8: O.MINE8}[md]
+
+    def problem():
+        pd = meshgen.uniform(n * 4, 1).reshape(n, 4)
+        w = meshgen.uniform(maps.shape[0] * 4, 2).reshape(4, -1)
+        return Problem([maps], [n], [pd.T.copy() if soa else pd], [w], bs, soa)
+
+    # a partition whose blocks come in another order than its cells
+    part = (np.arange(maps.shape[0]) // bs * 5 % 23).astype(np.uint32)
+    for partition in (None, part):
+        ref = _replay(problem(), k, bs, partition, 2)
+        for flags in (0, TP):
+            p = problem()
+            p.partition_vector = partition
+            p.gpu_loop(capi.functor(capi.KERNEL_MINE, md, 4, 4), capi.STRATEGY_HIERARCHICAL, 2,
+                       flags=flags)
+            assert_bitwise(p.point_data[0], ref, f"{kind} flags {flags}")
 
 
 @pytest.mark.parametrize("soa", [False, True])
