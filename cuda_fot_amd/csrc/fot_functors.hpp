@@ -608,6 +608,9 @@ template <int SLOT> struct LdsArgs {
   FOT_DEV uint32_t cs() const { return a.cs(); }
 };
 
+// The cell data slot a functor writes, or -1.
+template <class F> constexpr int kCellOutput = std::is_same_v<F, LuleshF> ? 1 : -1;
+
 // Staged input as rows of a constant, odd number of values per point: a
 // point's values sit at immediate offsets (two to an LDS read), and rows
 // start in different banks.
@@ -617,16 +620,15 @@ template <class F> struct StagedRows {
 
 // The engine arguments seen by a functor's SOA form whose staged input is in
 // LDS rows and whose cell data 0 is in registers: `tgt` holds block-local ids
-// times the row, a point's values are one apart, and so are the cell's; other
-// cell data is the caller's at the cell's position (`ind` is 0).
+// times the row, a point's values are one apart, and so are the cell's; its
+// cell output goes to `cell_out` (`ind` is 0).
 template <int SLOT> struct LdsRows {
   const EngineArgs &a;
-  const double *staged, *cell;
-  uint32_t pos;
+  const double *staged, *cell, *cell_out;
   static constexpr bool kStreamCells = false;
   FOT_DEV const double *pd(uint32_t k) const { return k == uint32_t(SLOT) ? staged : a.pd(k); }
   FOT_DEV uint32_t ps(uint32_t k) const { return k == uint32_t(SLOT) ? 1u : a.ps(k); }
-  FOT_DEV const double *cd(uint32_t k) const { return k == 0 ? cell : a.cd(k) + pos; }
+  FOT_DEV const double *cd(uint32_t k) const { return k == 0 ? cell : cell_out; }
   FOT_DEV uint32_t cs() const { return 1u; }
 };
 

@@ -56,9 +56,24 @@ struct HierDev {
   const uint4 *rec;
   const uint32_t *lists;
   uint32_t wide;
+  const uint32_t *cell_ids; // the caller's cell per position (cell outputs)
 };
 
 constexpr uint32_t kExclusive = 0xffffffffu;
+
+// Where a step's sums start from and go.  A plain step adds to the output in
+// place.  fot_loop_run's first and last step also do its copies: the first
+// starts from the iterate instead of a copy of it, and the last stores the
+// sums in the iterate too.  (mine 1024^2, 10 iterations, each with a copy of
+// 10.8 us in 54: 527 -> 365 us a call; lulesh 96^3, one iteration with two
+// copies of 9.7 us and the volumes' scatter of 7.8: 88 -> 68.)
+struct RunIO {
+  const double *base; // the values the increments are added to
+  double *out;
+  double *also;  // a second place for the sums, or null
+  double *cells; // the caller's array for the functor's cell output, or null
+                 // (then the plan-order copy)
+};
 
 // Two-phase writeback of a block's cache entry i (point g, values v): added
 // in place when this block alone touches g, else stored in its partial slot
@@ -87,7 +102,7 @@ FOT_DEV void writeback_two_phase(const HierDev &h, double *out, uint32_t np, uin
 // reads, measured 5 % slower on hex and mini_aero meshes.)
 template <uint32_t TD, bool SOA>
 __global__ __launch_bounds__(256) void merge_partials_kernel(
-    double *__restrict__ out, uint32_t np, const uint32_t *__restrict__ pt,
+    RunIO io, uint32_t np, const uint32_t *__restrict__ pt,
     const uint32_t *__restrict__ off, const uint32_t *__restrict__ slots,
     const double *__restrict__ partial, uint32_t n) {
   const uint32_t j = blockIdx.x * 256u + threadIdx.x;
@@ -95,14 +110,18 @@ __global__ __launch_bounds__(256) void merge_partials_kernel(
   const uint32_t g = pt[j], s0 = off[j], s1 = off[j + 1];
   double v[TD];
 #pragma unroll
-  for (uint32_t d = 0; d < TD; ++d) v[d] = out[pidx<SOA>(np, g, TD, d)];
+  for (uint32_t d = 0; d < TD; ++d) v[d] = io.base[pidx<SOA>(np, g, TD, d)];
   for (uint32_t s = s0; s < s1; ++s) {
     const double *q = partial + size_t(slots[s]) * TD;
 #pragma unroll
     for (uint32_t d = 0; d < TD; ++d) v[d] = v[d] + q[d];
   }
 #pragma unroll
-  for (uint32_t d = 0; d < TD; ++d) out[pidx<SOA>(np, g, TD, d)] = v[d];
+  for (uint32_t d = 0; d < TD; ++d) io.out[pidx<SOA>(np, g, TD, d)] = v[d];
+  if (io.also) {
+#pragma unroll
+    for (uint32_t d = 0; d < TD; ++d) io.also[pidx<SOA>(np, g, TD, d)] = v[d];
+  }
 }
 
 template <uint32_t MD>
@@ -535,8 +554,8 @@ template <class F, bool SOA> struct RowIds {
 // place.
 template <class F, bool SOA, int R, int LB = 1024, bool NTC = false>
 __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_gather_kernel(
-    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, uint32_t blk_begin,
-    uint32_t nbc) {
+    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, RunIO io,
+    uint32_t blk_begin, uint32_t nbc) {
   constexpr uint32_t MD = F::MD, TD = F::TD, PD = std::min(kPassDims<F>, TD);
   extern __shared__ double lds[];
   const uint4 rec = h.rec[blk_begin + xcd_block(blockIdx.x, nbc)];
@@ -572,6 +591,10 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_g
 #pragma unroll
     for (uint32_t k = 0; k < SI::cell_dim; ++k)
       cell[k] = load_once<NTC>(&a.cd(0)[pos + size_t(k) * a.cs()]);
+    double *cell_out = nullptr;
+    if constexpr (kCellOutput<F> >= 0)
+      cell_out = io.cells ? io.cells + h.cell_ids[pos]
+                          : const_cast<double *>(a.cd(kCellOutput<F>)) + pos;
     const double *src = a.pd(SI::slot);
     const uint32_t n = a.ps(SI::slot);
     constexpr uint32_t row = StagedRows<F>::row;
@@ -597,7 +620,7 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_g
 #pragma unroll
     for (uint32_t k = 0; k < MD; ++k) tgt[k] *= row;
     __syncthreads();
-    if (tid < ne) F::template compute<true>(LdsRows<SI::slot>{a, lds, cell, pos}, 0, tgt, inc);
+    if (tid < ne) F::template compute<true>(LdsRows<SI::slot>{a, lds, cell, cell_out}, 0, tgt, inc);
     __syncthreads(); // the planes take the staged values' place
   } else {
     if constexpr (kNeedsTargets<F>) targets<F>(a, pos, tgt);
@@ -644,9 +667,13 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_g
     if (slot[r] == kExclusive) {
       double o[TD];
 #pragma unroll
-      for (uint32_t d = 0; d < TD; ++d) o[d] = a.out[pidx<SOA>(np, g[r], TD, d)];
+      for (uint32_t d = 0; d < TD; ++d) o[d] = io.base[pidx<SOA>(np, g[r], TD, d)];
 #pragma unroll
-      for (uint32_t d = 0; d < TD; ++d) a.out[pidx<SOA>(np, g[r], TD, d)] = o[d] + v[r][d];
+      for (uint32_t d = 0; d < TD; ++d) io.out[pidx<SOA>(np, g[r], TD, d)] = o[d] + v[r][d];
+      if (io.also) {
+#pragma unroll
+        for (uint32_t d = 0; d < TD; ++d) io.also[pidx<SOA>(np, g[r], TD, d)] = o[d] + v[r][d];
+      }
     } else {
 #pragma unroll
       for (uint32_t d = 0; d < TD; ++d) h.partial[size_t(slot[r]) * TD + d] = v[r][d];
@@ -785,8 +812,8 @@ template <class F>
 constexpr bool kEarlyStaging = !std::is_same_v<F, fot::MiniAeroF> && !std::is_same_v<F, fot::GetaccF>;
 
 template <class F, bool SOA>
-__device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &h, uint32_t b,
-                                            double *lds) {
+__device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &h,
+                                            const RunIO &io, uint32_t b, double *lds) {
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
   const uint32_t e0 = h.blk_cell_off[b], ne = h.blk_cell_off[b + 1] - e0;
   const uint32_t c0 = h.blk_cache_off[b];
@@ -816,7 +843,7 @@ __device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &
     for (uint32_t k = 0; k < F::MD; ++k) loc[k] = cells ? loc[k] : 0u;
     double v0[F::TD];
 #pragma unroll
-    for (uint32_t d = 0; d < F::TD; ++d) v0[d] = a.out[pidx<SOA>(np, g0, F::TD, d)];
+    for (uint32_t d = 0; d < F::TD; ++d) v0[d] = io.base[pidx<SOA>(np, g0, F::TD, d)];
 #pragma unroll
     for (uint32_t k = 0; k < F::MD; ++k) tgt[k] = h.cached[c0 + loc[k]];
     if (tid < nw) {
@@ -828,7 +855,7 @@ __device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &
       const uint32_t g = h.cached[c0 + i];
       g_s[i] = g;
 #pragma unroll
-      for (uint32_t d = 0; d < F::TD; ++d) cache[d * nw + i] = a.out[pidx<SOA>(np, g, F::TD, d)];
+      for (uint32_t d = 0; d < F::TD; ++d) cache[d * nw + i] = io.base[pidx<SOA>(np, g, F::TD, d)];
     }
     if (tid < ne) {
       colour = colour_c;
@@ -840,7 +867,7 @@ __device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &
       const uint32_t g = h.cached[c0 + i];
       g_s[i] = g;
 #pragma unroll
-      for (uint32_t d = 0; d < F::TD; ++d) cache[d * nw + i] = a.out[pidx<SOA>(np, g, F::TD, d)];
+      for (uint32_t d = 0; d < F::TD; ++d) cache[d * nw + i] = io.base[pidx<SOA>(np, g, F::TD, d)];
     }
     if (tid < ne) {
       const uint32_t pos = e0 + tid;
@@ -860,14 +887,19 @@ __device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &
   for (uint32_t i = tid; i < nw; i += blockDim.x) {
     const uint32_t g = g_s[i];
 #pragma unroll
-    for (uint32_t d = 0; d < F::TD; ++d) a.out[pidx<SOA>(np, g, F::TD, d)] = cache[d * nw + i];
+    for (uint32_t d = 0; d < F::TD; ++d) io.out[pidx<SOA>(np, g, F::TD, d)] = cache[d * nw + i];
+    if (io.also) {
+#pragma unroll
+      for (uint32_t d = 0; d < F::TD; ++d) io.also[pidx<SOA>(np, g, F::TD, d)] = cache[d * nw + i];
+    }
   }
 }
 
 template <class F, bool SOA, int LB = 1024>
-__global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, uint32_t nb) {
+__global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, RunIO io,
+                                                       uint32_t nb) {
   extern __shared__ double lds[];
-  owner_block<F, SOA>(a, h, xcd_block(blockIdx.x, nb), lds);
+  owner_block<F, SOA>(a, h, io, xcd_block(blockIdx.x, nb), lds);
 }
 
 // One problem of a batch: its engine arguments and owner-compute plan.
@@ -885,7 +917,8 @@ template <class F, bool SOA>
 __global__ __launch_bounds__(1024) void batch_owner_kernel(const BatchProblem *__restrict__ probs,
                                                            const uint2 *__restrict__ work,
                                                            uint32_t nwork,
-                                                           uint32_t *__restrict__ queue) {
+                                                           uint32_t *__restrict__ queue,
+                                                           bool from_iterate, bool to_iterate) {
   extern __shared__ double lds[];
   // the next item is taken while the current one runs, so the queue
   // atomic's round trip overlaps the work instead of preceding each item
@@ -896,7 +929,10 @@ __global__ __launch_bounds__(1024) void batch_owner_kernel(const BatchProblem *_
   while (w < nwork) {
     if (threadIdx.x == 0) item[buf ^ 1u] = atomicAdd(&queue[0], 1u);
     const uint2 pb = work[w];
-    owner_block<F, SOA>(probs[pb.x].args, probs[pb.x].hier, pb.y, lds);
+    const EngineArgs &a = probs[pb.x].args;
+    double *iterate = const_cast<double *>(a.point_data[0]);
+    const RunIO io{from_iterate ? iterate : a.out, a.out, to_iterate ? iterate : nullptr, nullptr};
+    owner_block<F, SOA>(a, probs[pb.x].hier, io, pb.y, lds);
     __syncthreads(); // this item's LDS no longer read; the next index visible
     buf ^= 1u;
     w = item[buf];
@@ -1190,8 +1226,8 @@ FOT_DEV void owner3_load_ids(Owner3Ids<EPT, KS, KO> &id, const OwnerMeta &mt, co
 // read again
 template <bool SOA, int EPT, int KS, int KO, bool NT = false>
 FOT_DEV void owner3_load_data(Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, KS, KO> &id,
-                              const OwnerMeta &mt, const EngineArgs &a, uint32_t tid,
-                              uint32_t bd) {
+                              const OwnerMeta &mt, const EngineArgs &a, const RunIO &io,
+                              uint32_t tid, uint32_t bd) {
   const double *x = a.point_data[1], *q = a.point_data[2], *adt = a.point_data[3];
   const uint32_t np = a.num_points[0], nw = mt.nowned;
 #pragma unroll
@@ -1206,8 +1242,8 @@ FOT_DEV void owner3_load_data(Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, K
         double r[4];
 #pragma unroll
         for (uint32_t c = 0; c < 4; ++c)
-          r[c] = NT ? __builtin_nontemporal_load(&a.out[c * size_t(np) + gr])
-                    : a.out[c * size_t(np) + gr];
+          r[c] = NT ? __builtin_nontemporal_load(&io.base[c * size_t(np) + gr])
+                    : io.base[c * size_t(np) + gr];
         d.vr0[k] = make_double2(r[0], r[1]), d.vr1[k] = make_double2(r[2], r[3]);
       }
     } else {
@@ -1215,11 +1251,11 @@ FOT_DEV void owner3_load_data(Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, K
       d.vq0[k] = q2p[2 * size_t(g)], d.vq1[k] = q2p[2 * size_t(g) + 1];
       if (k < KO) {
         if (NT) {
-          const dvec2 *o = reinterpret_cast<const dvec2 *>(a.out) + 2 * size_t(gr);
+          const dvec2 *o = reinterpret_cast<const dvec2 *>(io.base) + 2 * size_t(gr);
           const dvec2 r0 = __builtin_nontemporal_load(o), r1 = __builtin_nontemporal_load(o + 1);
           d.vr0[k] = make_double2(r0.x, r0.y), d.vr1[k] = make_double2(r1.x, r1.y);
         } else {
-          const double2 *o = reinterpret_cast<const double2 *>(a.out) + 2 * size_t(gr);
+          const double2 *o = reinterpret_cast<const double2 *>(io.base) + 2 * size_t(gr);
           d.vr0[k] = o[0], d.vr1[k] = o[1];
         }
       }
@@ -1240,6 +1276,28 @@ FOT_DEV void owner3_load_data(Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, K
   }
 }
 
+// one cell's sums to an output
+template <bool SOA, bool NT>
+FOT_DEV void owner3_store(double *out, uint32_t np, uint32_t g, const double *r) {
+  if (SOA) {
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+      if (NT)
+        __builtin_nontemporal_store(r[c], &out[size_t(c) * np + g]);
+      else
+        out[size_t(c) * np + g] = r[c];
+    }
+  } else if (NT) {
+    dvec2 *o = reinterpret_cast<dvec2 *>(out) + 2 * size_t(g);
+    __builtin_nontemporal_store(dvec2{r[0], r[1]}, o);
+    __builtin_nontemporal_store(dvec2{r[2], r[3]}, o + 1);
+  } else {
+    double2 *o = reinterpret_cast<double2 *>(out) + 2 * size_t(g);
+    o[0] = make_double2(r[0], r[1]);
+    o[1] = make_double2(r[2], r[3]);
+  }
+}
+
 // stage q / adt, fluxes, gather, store.  Starts with the LDS free; ends with
 // the LDS still being read by other waves (callers reusing it sync first).
 // With PRE, 1/rho and the pressure of each staged cell are computed once at
@@ -1247,7 +1305,8 @@ FOT_DEV void owner3_load_data(Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, K
 // same values, the same bits.
 template <bool SOA, int EPT, int KS, int LW, int KO, bool PRE, bool NT = false>
 FOT_DEV void owner3_body(double *lds, Owner3Data<EPT, KS, KO> &d, const Owner3Ids<EPT, KS, KO> &id,
-                         const OwnerMeta &mt, const EngineArgs &a, uint32_t tid, uint32_t bd) {
+                         const OwnerMeta &mt, const EngineArgs &a, const RunIO &io, uint32_t tid,
+                         uint32_t bd) {
   const uint32_t m = mt.ncached, nw = mt.nowned, ne = mt.ncells;
   const uint32_t np = a.num_points[0];
   // LDS holds double2 planes, so lanes on consecutive slots touch
@@ -1346,23 +1405,8 @@ FOT_DEV void owner3_body(double *lds, Owner3Data<EPT, KS, KO> &d, const Owner3Id
         }
       }
       const uint32_t g = id.gq[k];
-      if (SOA) {
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-          if (NT)
-            __builtin_nontemporal_store(r[c], &a.out[size_t(c) * np + g]);
-          else
-            a.out[size_t(c) * np + g] = r[c];
-        }
-      } else if (NT) {
-        dvec2 *o = reinterpret_cast<dvec2 *>(a.out) + 2 * size_t(g);
-        __builtin_nontemporal_store(dvec2{r[0], r[1]}, o);
-        __builtin_nontemporal_store(dvec2{r[2], r[3]}, o + 1);
-      } else {
-        double2 *o = reinterpret_cast<double2 *>(a.out) + 2 * size_t(g);
-        o[0] = make_double2(r[0], r[1]);
-        o[1] = make_double2(r[2], r[3]);
-      }
+      owner3_store<SOA, NT>(io.out, np, g, r);
+      if (io.also) owner3_store<SOA, NT>(io.also, np, g, r);
     }
   }
 }
@@ -1373,7 +1417,7 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
                                                                const uint32_t *__restrict__ cached,
                                                                const uint32_t *__restrict__ packed,
                                                                const uint32_t *__restrict__ plist,
-                                                               uint32_t nb) {
+                                                               RunIO io, uint32_t nb) {
   extern __shared__ double lds[];
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
@@ -1381,8 +1425,8 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
   Owner3Ids<EPT, KS, KO> id;
   Owner3Data<EPT, KS, KO> d;
   owner3_load_ids<EPT, KS, LW, KO>(id, mt, a, cached, packed, plist, tid, bd);
-  owner3_load_data<SOA, EPT, KS, KO>(d, id, mt, a, tid, bd);
-  owner3_body<SOA, EPT, KS, LW, KO, PRE>(lds, d, id, mt, a, tid, bd);
+  owner3_load_data<SOA, EPT, KS, KO>(d, id, mt, a, io, tid, bd);
+  owner3_body<SOA, EPT, KS, LW, KO, PRE>(lds, d, id, mt, a, io, tid, bd);
 }
 
 // The same with the owned res loaded and stored nontemporally (edge lists
@@ -1390,7 +1434,8 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
 template <bool SOA, int EPT, int KS, int KO>
 __global__ __launch_bounds__(1024) void res_calc_owner3_stream_kernel(
     EngineArgs a, const OwnerMeta *__restrict__ meta, const uint32_t *__restrict__ cached,
-    const uint32_t *__restrict__ packed, const uint32_t *__restrict__ plist, uint32_t nb) {
+    const uint32_t *__restrict__ packed, const uint32_t *__restrict__ plist, RunIO io,
+    uint32_t nb) {
   extern __shared__ double lds[];
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
@@ -1398,8 +1443,8 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_stream_kernel(
   Owner3Ids<EPT, KS, KO> id;
   Owner3Data<EPT, KS, KO> d;
   owner3_load_ids<EPT, KS, 0, KO>(id, mt, a, cached, packed, plist, tid, bd);
-  owner3_load_data<SOA, EPT, KS, KO, true>(d, id, mt, a, tid, bd);
-  owner3_body<SOA, EPT, KS, 0, KO, false, true>(lds, d, id, mt, a, tid, bd);
+  owner3_load_data<SOA, EPT, KS, KO, true>(d, id, mt, a, io, tid, bd);
+  owner3_body<SOA, EPT, KS, 0, KO, false, true>(lds, d, id, mt, a, io, tid, bd);
 }
 
 // Persistent form: gridDim.x workgroups (a multiple of 8, at most the
@@ -1414,7 +1459,7 @@ __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
                                                                const uint32_t *__restrict__ cached,
                                                                const uint32_t *__restrict__ packed,
                                                                const uint32_t *__restrict__ plist,
-                                                               uint32_t nb) {
+                                                               RunIO io, uint32_t nb) {
   extern __shared__ double lds[];
   const uint32_t tid = threadIdx.x, bd = blockDim.x, G = gridDim.x;
   uint32_t j = blockIdx.x;
@@ -1424,14 +1469,14 @@ __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
   owner3_load_ids<EPT, KS, LW, KO>(id, mt, a, cached, packed, plist, tid, bd);
   for (;;) {
     Owner3Data<EPT, KS, KO> d;
-    owner3_load_data<SOA, EPT, KS, KO>(d, id, mt, a, tid, bd);
+    owner3_load_data<SOA, EPT, KS, KO>(d, id, mt, a, io, tid, bd);
     const uint32_t jn = j + G;
     const bool more = jn < nb; // uniform
     // the last block loads its own entries again: branch-free, in bounds
     const OwnerMeta mtn = meta[xcd_block(more ? jn : j, nb)];
     Owner3Ids<EPT, KS, KO> idn;
     owner3_load_ids<EPT, KS, LW, KO>(idn, mtn, a, cached, packed, plist, tid, bd);
-    owner3_body<SOA, EPT, KS, LW, KO, PRE>(lds, d, id, mt, a, tid, bd);
+    owner3_body<SOA, EPT, KS, LW, KO, PRE>(lds, d, id, mt, a, io, tid, bd);
     if (!more) break;
     __syncthreads(); // the next block's staging overwrites f_s
     j = jn;
@@ -1573,8 +1618,8 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
 // Launches eng_gather_kernel<F, SOA, R>.
 template <class F, bool SOA, int R>
 void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
-                   const EngineArgs &a, const HierDev &h, uint32_t b0, uint32_t nbc,
-                   bool stream_cells) {
+                   const EngineArgs &a, const HierDev &h, const RunIO &io, uint32_t b0,
+                   uint32_t nbc, bool stream_cells) {
   constexpr int SB = kSmallBound<F>;
   const bool small = threads <= uint32_t(SB);
   if constexpr (kStreamsCells<F>) {
@@ -1582,19 +1627,19 @@ void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
       const StreamCellArgs sa{a};
       if (small)
         hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB, true>), dim3(grid), dim3(threads),
-                           lds, s, sa, h, b0, nbc);
+                           lds, s, sa, h, io, b0, nbc);
       else
         hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, 1024, true>), dim3(grid), dim3(threads),
-                           lds, s, sa, h, b0, nbc);
+                           lds, s, sa, h, io, b0, nbc);
       return;
     }
   }
   if (small)
     hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB>), dim3(grid), dim3(threads), lds, s, a, h,
-                       b0, nbc);
+                       io, b0, nbc);
   else
     hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R>), dim3(grid), dim3(threads), lds, s, a, h,
-                       b0, nbc);
+                       io, b0, nbc);
 }
 
 // Values per point of a functor's staged input (0: none).
@@ -1767,7 +1812,16 @@ struct fot_loop {
   fot_status build_atomic();
   fot_status build_global_colour();
   fot_status build_hierarchical();
-  fot_status enqueue(hipStream_t s);
+  // one step, adding in place, or as `run` says (where fuses_run allows it)
+  fot_status enqueue(hipStream_t s, const RunIO *run = nullptr);
+  // whether fot_loop_run's copies can be part of its first and last step
+  bool fuses_run() const;
+  // whether none of its point arrays overlaps the n values at p
+  bool keeps_off(const double *p, uint64_t n) const;
+  static bool overlaps(const double *p, uint64_t n, const double *q, uint64_t m) {
+    return p && q && p < q + m && q < p + n;
+  }
+  bool every_point = false; // a step writes every point of mapping 0
 };
 
 fot_status fot_loop::build_atomic() {
@@ -1957,6 +2011,10 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
     if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
     hier.loc = d16;
   }
+  if (cell_output_slot(f) >= 0) {
+    if ((st = upload(plan_cell.data(), plan_cell.size(), &d32)) != FOT_OK) return st;
+    hier.cell_ids = d32;
+  }
   lds_bytes = lds;
   gather = true;
   return FOT_OK;
@@ -2106,6 +2164,8 @@ fot_status fot_loop::build_hierarchical() {
   if ((st = upload(cached.data(), cached.size(), &d32)) != FOT_OK) return st;
   hier.cached = d32;
   if (owner) {
+    every_point = std::accumulate(blk_owned.begin(), blk_owned.end(), uint64_t(0)) ==
+                  desc.num_points[0];
     if ((st = upload(blk_owned.data(), blk_owned.size(), &d32)) != FOT_OK) return st;
     hier.blk_owned = d32;
     if (f.kernel == FOT_KERNEL_RES_CALC) {
@@ -2264,6 +2324,7 @@ fot_status fot_loop::build_hierarchical() {
           const uint32_t r = rank[cached[i]];
           slots[off[r] + fill[r]++] = wslot[i];
         }
+    every_point = std::find(touch.begin(), touch.end(), 0u) == touch.end();
     merge_n = uint32_t(pt.size());
     if ((st = upload(wslot.data(), wslot.size(), &d32)) != FOT_OK) return st;
     hier.wslot = d32;
@@ -2475,8 +2536,9 @@ template <class F> uint32_t atomic_threads(uint32_t cells) {
   return n;
 }
 
-fot_status fot_loop::enqueue(hipStream_t s) {
+fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
   if (desc.num_cells == 0) return FOT_OK; // nothing to launch
+  const RunIO io = run ? *run : RunIO{base.out, base.out, nullptr, nullptr};
   const fot_status st = dispatch(&f, desc.soa, [&]<class F, bool SOA>() -> fot_status {
     const uint32_t bs = cfg.block_size;
     // direct launches: one thread per cell, whatever the block size
@@ -2523,7 +2585,8 @@ fot_status fot_loop::enqueue(hipStream_t s) {
           const OwnerMeta *om = owner_meta;
           const uint32_t *pc = hier.cached, *pp = hier.packed, *pl = owner_plist;
           uint32_t nbv = nb;
-          void *kargs[] = {&pa, &om, &pc, &pp, &pl, &nbv};
+          RunIO iov = io;
+          void *kargs[] = {&pa, &om, &pc, &pp, &pl, &iov, &nbv};
           FOT_HIP(hipLaunchKernel(owner3_fn, dim3(launch_grid), dim3(threads), kargs,
                                   size_t(lds_bytes), s));
         } else if (ept == 2) {
@@ -2541,13 +2604,13 @@ fot_status fot_loop::enqueue(hipStream_t s) {
         if constexpr (kSmallBound<F> < 1024) {
           if (threads <= uint32_t(kSmallBound<F>)) {
             hipLaunchKernelGGL((eng_owner_kernel<F, SOA, kSmallBound<F>>), dim3(nb), dim3(threads),
-                               lds_bytes, s, plan_args, hier, nb);
+                               lds_bytes, s, plan_args, hier, io, nb);
             done = true;
           }
         }
         if (!done)
           hipLaunchKernelGGL((eng_owner_kernel<F, SOA>), dim3(nb), dim3(threads), lds_bytes, s,
-                             plan_args, hier, nb);
+                             plan_args, hier, io, nb);
       }
     } else if (dep_order) {
       // one launch over every plan block
@@ -2576,15 +2639,15 @@ fot_status fot_loop::enqueue(hipStream_t s) {
       }
       if (gather) {
         if (gather_rounds == 1)
-          launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, 0u, nb, nontemporal);
+          launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, io, 0u, nb, nontemporal);
         else
-          launch_gather<F, SOA, 2>(nb, threads, lds_bytes, s, plan_args, hier, 0u, nb, nontemporal);
+          launch_gather<F, SOA, 2>(nb, threads, lds_bytes, s, plan_args, hier, io, 0u, nb, nontemporal);
       } else if (!done)
         launch_eng_hier<F, SOA, 2>(stage_pd, nb, threads, lds_bytes, s, plan_args, hier, dep,
                                    0u, nb, nontemporal);
       if (merge_n)
         hipLaunchKernelGGL((merge_partials_kernel<F::TD, SOA>), dim3((merge_n + 255) / 256),
-                           dim3(256), 0, s, plan_args.out, plan_args.num_points[0], merge_pt,
+                           dim3(256), 0, s, io, plan_args.num_points[0], merge_pt,
                            merge_off, merge_slots, hier.partial, merge_n);
     } else {
       for (size_t c = 0; c + 1 < colour_blk_off.size(); ++c) {
@@ -2598,9 +2661,9 @@ fot_status fot_loop::enqueue(hipStream_t s) {
           }
         }
         if (gather && gather_rounds == 1)
-          launch_gather<F, SOA, 1>(nbc, threads, lds_bytes, s, plan_args, hier, b0, nbc, false);
+          launch_gather<F, SOA, 1>(nbc, threads, lds_bytes, s, plan_args, hier, io, b0, nbc, false);
         else if (gather)
-          launch_gather<F, SOA, 2>(nbc, threads, lds_bytes, s, plan_args, hier, b0, nbc, false);
+          launch_gather<F, SOA, 2>(nbc, threads, lds_bytes, s, plan_args, hier, io, b0, nbc, false);
         else
           launch_eng_hier<F, SOA, 0>(stage_pd, nbc, threads, lds_bytes, s, plan_args, hier, dep,
                                    b0, nbc);
@@ -2760,14 +2823,64 @@ extern "C" fot_status fot_loop_step(fot_loop *loop, void *stream) {
   return fot::guarded("fot_loop_step", [&] { return fot_loop_step_impl(loop, stream); });
 }
 
+bool fot_loop::fuses_run() const {
+  // every point has to be written by the step that replaces a copy, by a kernel
+  // that takes a RunIO; a captured graph's steps add in place
+  if (exec || desc.num_cells == 0 || !every_point) return false;
+  const bool jacobi = reads_iterate(f);
+  if (!(two_phase && gather) &&
+      !(owner && !jacobi && (f.kernel != FOT_KERNEL_RES_CALC || owner_gather)))
+    return false;
+  // and the iterate is nobody else's: not the output, no other input
+  const double *in = desc.point_data[0];
+  const uint64_t n = uint64_t(desc.num_points[0]) * desc.point_dim[0];
+  for (uint32_t k = 1; k < desc.num_mappings; ++k)
+    if (overlaps(in, n, desc.point_data[k], uint64_t(desc.num_points[k]) * desc.point_dim[k]))
+      return false;
+  const int slot = cell_output_slot(f);
+  if (slot >= 0 && overlaps(in, n, desc.cell_data[slot],
+                            uint64_t(desc.num_cells) * desc.cell_dim[slot]))
+    return false;
+  return !overlaps(in, n, base.out, n);
+}
+
+bool fot_loop::keeps_off(const double *p, uint64_t n) const {
+  if (overlaps(p, n, base.out, uint64_t(desc.num_points[0]) * desc.point_dim[0])) return false;
+  for (uint32_t k = 0; k < desc.num_mappings; ++k)
+    if (overlaps(p, n, desc.point_data[k], uint64_t(desc.num_points[k]) * desc.point_dim[k]))
+      return false;
+  return true;
+}
+
 static fot_status fot_loop_run_impl(fot_loop *loop, uint32_t iters, void *stream) {
   if (!loop) return fail(FOT_ERR_INVALID_ARGUMENT, "null loop");
   const fot_problem_desc &d = loop->desc;
   double *in = const_cast<double *>(d.point_data[0]);
   const size_t bytes = sizeof(double) * size_t(d.num_points[0]) * d.point_dim[0];
-  fot_status st = fot_copy(d.point_data_out, in, bytes, stream);
-  if (st != FOT_OK) return st;
+  const hipStream_t hs = static_cast<hipStream_t>(stream);
   const bool jacobi = reads_iterate(loop->f);
+  fot_status st;
+  if (iters && loop->fuses_run()) {
+    // The first step starts from the iterate; the last stores its sums there
+    // too.  A functor that reads its iterate works on it in place (a two-phase
+    // block writes only points that no other block reads, and the merge runs
+    // when every block has read), and the output gets the last step's.
+    const int slot = cell_output_slot(loop->f);
+    for (uint32_t it = 0; it < iters; ++it) {
+      const bool last = it + 1 == iters;
+      RunIO io{it == 0 || jacobi ? in : d.point_data_out, d.point_data_out, last ? in : nullptr,
+               nullptr};
+      if (jacobi) io.out = in, io.also = last ? d.point_data_out : nullptr;
+      if (last && slot >= 0 && loop->hier.cell_ids)
+        io.cells = const_cast<double *>(d.cell_data[slot]);
+      if ((st = loop->enqueue(hs, &io)) != FOT_OK) return st;
+    }
+    if (!loop->hier.cell_ids && (st = loop->scatter_cell_outputs(hs)) != FOT_OK) return st;
+    FOT_HIP(hipStreamSynchronize(hs));
+    return FOT_OK;
+  }
+  st = fot_copy(d.point_data_out, in, bytes, stream);
+  if (st != FOT_OK) return st;
   for (uint32_t it = 0; it < iters; ++it) {
     if ((st = fot_loop_step(loop, stream)) != FOT_OK) return st;
     if (jacobi || it + 1 == iters)
@@ -2838,11 +2951,13 @@ struct fot_batch {
     *dev = static_cast<T *>(p);
     return FOT_OK;
   }
-  fot_status launch_step(hipStream_t s) {
+  // whether fot_batch_run's copies are part of its first and last step
+  bool fused = false;
+  fot_status launch_step(hipStream_t s, bool from_iterate = false, bool to_iterate = false) {
     if (nwork == 0) return FOT_OK;
     return dispatch(&f, soa, [&]<class F, bool SOA>() -> fot_status {
       hipLaunchKernelGGL((batch_owner_kernel<F, SOA>), dim3(grid), dim3(threads), lds_bytes, s,
-                         probs, work, nwork, queue);
+                         probs, work, nwork, queue, from_iterate, to_iterate);
       FOT_HIP(hipGetLastError());
       return FOT_OK;
     });
@@ -2890,6 +3005,15 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
       cin.push_back({descs[i].point_data_out + o, in + o, cnt, 0});
       cback.push_back({in + o, descs[i].point_data_out + o, cnt, 0});
     }
+  }
+  B->fused = !use_graph;
+  for (uint32_t i = 0; i < num_problems && B->fused; ++i) {
+    B->fused = B->loops[i]->fuses_run();
+    // ... and no other problem has this one's iterate
+    for (uint32_t j = 0; j < num_problems && B->fused; ++j)
+      B->fused = i == j || B->loops[j]->keeps_off(descs[i].point_data[0],
+                                                  uint64_t(descs[i].num_points[0]) *
+                                                      descs[i].point_dim[0]);
   }
   // work items, largest problems first (longest jobs first balances the tail)
   std::vector<uint32_t> order(num_problems);
@@ -2973,7 +3097,17 @@ extern "C" fot_status fot_batch_step(fot_batch *b, void *stream) {
 static fot_status fot_batch_run_impl(fot_batch *b, uint32_t iters, void *stream) {
   if (!b) return fail(FOT_ERR_INVALID_ARGUMENT, "null batch");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  fot_status st = b->launch_copy(b->copy_in, s);
+  fot_status st = FOT_OK;
+  if (iters && b->fused) {
+    for (uint32_t it = 0; it < iters && st == FOT_OK; ++it)
+      st = b->launch_step(s, it == 0, it + 1 == iters);
+    for (fot_loop *l : b->loops)
+      if (st == FOT_OK) st = l->scatter_cell_outputs(s);
+    if (st != FOT_OK) return st;
+    FOT_HIP(hipStreamSynchronize(s));
+    return FOT_OK;
+  }
+  st = b->launch_copy(b->copy_in, s);
   for (uint32_t it = 0; it < iters && st == FOT_OK; ++it) {
     if (b->exec) {
       FOT_HIP(hipGraphLaunch(b->exec, s)); // copies back itself when jacobi

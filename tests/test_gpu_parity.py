@@ -308,6 +308,46 @@ def test_gathered_sums_at_their_limits(gpu, kind, soa):
             assert_bitwise(p.point_data[0], ref, f"{kind} flags {flags}")
 
 
+@pytest.mark.parametrize("iters", [1, 2, 3])
+@pytest.mark.parametrize("isolated", [0, 3])
+@pytest.mark.parametrize("kind", ["mine two-phase", "hex two-phase", "hex owner", "airfoil owner"])
+def test_run_leaves_iterate_and_output_alike(gpu, kind, isolated, iters):
+    """run()'s copies are part of its first and last step where every point is
+    written: the iterate and the output hold the result either way, and as
+    steps with explicit copies give it."""
+    from cuda_fot_amd import DeviceArray, Loop
+    p = mine_problem() if "mine" in kind else hex_problem() if "hex" in kind else \
+        airfoil_problem(res0_seed=5)
+    f = capi.functor(capi.KERNEL_MINE, 2, 4, 4) if "mine" in kind else \
+        capi.functor(capi.KERNEL_HEX_SCATTER) if "hex" in kind else RES_CALC
+    if isolated:  # points of mapping 0's set that no cell names
+        for k in range(len(p.maps)):
+            if p.num_points[k] == p.num_points[0] and (k == 0 or "airfoil" in kind):
+                d = p.point_data[k]
+                p.point_data[k] = np.concatenate([d, np.full((isolated,) + d.shape[1:], 1.5)])
+        p.num_points = [n + isolated if n == p.num_points[0] else n for n in p.num_points]
+    flags = TP if "two" in kind else \
+        capi.LOOP_OWNER_COMPUTE | capi.LOOP_TWO_PER_THREAD | capi.LOOP_OWNER_GATHER
+    got = []
+    for whole in (True, False):
+        dev = [DeviceArray.from_host(d) for d in p.point_data]
+        out = DeviceArray.from_host(np.full_like(p.point_data[0], np.nan))
+        cells = [DeviceArray.from_host(c) for c in p.cell_data]
+        loop = Loop(f, p.maps, p.num_points, dev, out, cells, block_size=128, flags=flags)
+        if whole:
+            loop.run(iters)
+        else:
+            capi.call("fot_copy", out.ptr, dev[0].ptr, out.nbytes, None)
+            for i in range(iters):
+                loop.step()
+                if "mine" in kind or i + 1 == iters:
+                    capi.call("fot_copy", dev[0].ptr, out.ptr, out.nbytes, None)
+        got += [dev[0].download(), out.download()]
+        loop.close()
+    for g in got[:3]:
+        assert_bitwise(g, got[3], kind)
+
+
 @pytest.mark.parametrize("soa", [False, True])
 def test_hex_scatter_strategies(gpu, soa):
     f = capi.functor(capi.KERNEL_HEX_SCATTER)
