@@ -57,6 +57,18 @@ struct HierDev {
   const uint32_t *lists;
   uint32_t wide;
   const uint32_t *cell_ids; // the caller's cell per position (cell outputs)
+  // owner compute with gathered sums: block records; `lists` per owned point
+  // (places MD planes of `cap` cells apart), `cached` its ids
+  const struct OwnerItem *items;
+  uint32_t cap;
+};
+
+// One block of an owner-compute plan (of a batch's problem).
+struct OwnerItem {
+  uint32_t problem, cell0, ncells; // its cells' plan positions
+  uint32_t point0, npoints;        // its owned points' entries
+  uint32_t first;                  // their ids are first + i, or kExclusive: in `cached`
+  uint32_t pad0, pad1;
 };
 
 constexpr uint32_t kExclusive = 0xffffffffu;
@@ -895,6 +907,116 @@ __device__ __forceinline__ void owner_block(const EngineArgs &a, const HierDev &
   }
 }
 
+// The owner block whose points gather (see eng_gather_kernel): E cells and R
+// owned points per thread, a point's list applied to its value in thread-colour
+// order, the additions of owner_block in its order.  An item's record names
+// everything a block reads first (cells, lists, the owned values, whose ids
+// are consecutive on a mesh renumbered by its parts), so a block is three
+// round trips: record, ids and values, gathered values.  Two cells per thread
+// halve the workgroup, and twice as many take turns at each CU's barriers.
+// Colour loop / this, single mesh as a step: mine 1024^2 on parts of 256 38.0
+// / 31.7 us, getacc 1024^2 69.6 / 49.1, volna 900^2 quads on parts of 512 66 /
+// 61 (4.8 TB/s).  Points of more than 8 increments, parts of more than 512
+// points or 1024 cells and the functors with more registers to hold (8 nodes,
+// mini_aero) keep the colour loop.
+template <class F>
+constexpr bool kOwnerGathers = F::MD <= 4 && !std::is_same_v<F, fot::MiniAeroF> &&
+                               !std::is_same_v<F, fot::ResCalcF>;
+constexpr uint32_t kOwnerCells = 2;  // E
+constexpr uint32_t kOwnerPoints = 1; // R
+template <class F> constexpr uint32_t kOwnerPassDims = F::MD == 2 ? (F::TD < 2 ? F::TD : 2) : 1;
+template <class F> constexpr uint32_t owner_gather_lds(uint32_t cap) {
+  return 8u * kOwnerPassDims<F> * (F::MD * cap + 1);
+}
+
+template <class F, bool SOA>
+__device__ __forceinline__ void owner_gather_block(const EngineArgs &a, const HierDev &h,
+                                                   const RunIO &io, const OwnerItem &it,
+                                                   double *lds) {
+  constexpr uint32_t MD = F::MD, TD = F::TD, PD = kOwnerPassDims<F>;
+  constexpr uint32_t E = kOwnerCells, R = kOwnerPoints;
+  const uint32_t tid = threadIdx.x, T = blockDim.x, np = a.num_points[0];
+  uint32_t tgt[E][MD], pos[E], g[R];
+  uint4 list[R];
+#pragma unroll
+  for (uint32_t e = 0; e < E; ++e) {
+    // (a block whose points no cell touches has none: it reads position 0)
+    pos[e] = it.ncells ? it.cell0 + min(tid + e * T, it.ncells - 1) : 0u;
+    if constexpr (kNeedsTargets<F>) targets<F>(a, pos[e], tgt[e]);
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t i = min(tid + r * T, it.npoints - 1);
+    if (h.wide) {
+      list[r] = reinterpret_cast<const uint4 *>(h.lists)[it.point0 + i];
+    } else {
+      const uint2 w = reinterpret_cast<const uint2 *>(h.lists)[it.point0 + i];
+      list[r] = make_uint4(w.x, w.y, 0u, 0u);
+    }
+    g[r] = it.first != kExclusive ? it.first + i : h.cached[it.point0 + i];
+  }
+  double v[R][TD];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r)
+#pragma unroll
+    for (uint32_t d = 0; d < TD; ++d) v[r][d] = io.base[pidx<SOA>(np, g[r], TD, d)];
+  double inc[E][MD * TD];
+#pragma unroll
+  for (uint32_t e = 0; e < E; ++e) F::template compute<SOA>(a, pos[e], tgt[e], inc[e]);
+  const uint32_t stride = MD * h.cap + 1; // + a zero for empty places
+#pragma unroll
+  for (uint32_t d0 = 0; d0 < TD; d0 += PD) {
+    if (d0) __syncthreads();
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+      if (tid + e * T < it.ncells) {
+#pragma unroll
+        for (uint32_t p = 0; p < PD; ++p)
+          if (d0 + p < TD) {
+#pragma unroll
+            for (uint32_t k = 0; k < MD; ++k)
+              lds[p * stride + k * h.cap + tid + e * T] = inc[e][k * TD + d0 + p];
+          }
+      }
+    // x + -0.0 is x for every x, zeros of either sign included
+    if (tid < PD) lds[tid * stride + MD * h.cap] = -0.0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+      const uint32_t at[8] = {list[r].x & 0xffffu, list[r].x >> 16, list[r].y & 0xffffu,
+                              list[r].y >> 16,     list[r].z & 0xffffu, list[r].z >> 16,
+                              list[r].w & 0xffffu, list[r].w >> 16};
+#pragma unroll
+      for (uint32_t p = 0; p < PD; ++p) {
+        if (d0 + p >= TD) continue;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) v[r][d0 + p] += lds[p * stride + at[j]];
+        if (h.wide) {
+#pragma unroll
+          for (uint32_t j = 4; j < 8; ++j) v[r][d0 + p] += lds[p * stride + at[j]];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    if (tid + r * T >= it.npoints) continue;
+#pragma unroll
+    for (uint32_t d = 0; d < TD; ++d) io.out[pidx<SOA>(np, g[r], TD, d)] = v[r][d];
+    if (io.also) {
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) io.also[pidx<SOA>(np, g[r], TD, d)] = v[r][d];
+    }
+  }
+}
+
+template <class F, bool SOA>
+__global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, HierDev h, RunIO io,
+                                                               uint32_t nb) {
+  extern __shared__ double lds[];
+  owner_gather_block<F, SOA>(a, h, io, h.items[xcd_block(blockIdx.x, nb)], lds);
+}
+
 template <class F, bool SOA, int LB = 1024>
 __global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, RunIO io,
                                                        uint32_t nb) {
@@ -907,6 +1029,30 @@ struct BatchProblem {
   EngineArgs args;
   HierDev hier;
 };
+
+// A pointer read from memory, as one to global memory.  The compiler takes
+// kernel arguments to be that by themselves; through any other pointer it
+// emits flat loads, which may be LDS and so can only be waited for all at once
+// (one after the other, that is, within a block's chain).
+template <class T> FOT_DEV T *as_global(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)reinterpret_cast<uintptr_t>(p);
+}
+FOT_DEV BatchProblem as_global(const BatchProblem &from) {
+  BatchProblem p = from;
+#pragma unroll
+  for (uint32_t k = 0; k < FOT_MAX_MAPPINGS; ++k)
+    p.args.point_data[k] = as_global(p.args.point_data[k]), p.args.maps[k] = as_global(p.args.maps[k]);
+#pragma unroll
+  for (uint32_t k = 0; k < FOT_MAX_CELL_DATA; ++k)
+    p.args.cell_data[k] = as_global(p.args.cell_data[k]);
+  p.args.out = as_global(p.args.out);
+  HierDev &h = p.hier;
+  h.blk_cell_off = as_global(h.blk_cell_off), h.blk_cache_off = as_global(h.blk_cache_off);
+  h.blk_owned = as_global(h.blk_owned), h.blk_ncol = as_global(h.blk_ncol);
+  h.cached = as_global(h.cached), h.loc = as_global(h.loc), h.colour = as_global(h.colour);
+  h.lists = as_global(h.lists);
+  return p;
+}
 
 // Batched owner-compute step: a persistent grid whose workgroups take
 // (problem, block) items from a device queue until it runs dry.  queue[0] is
@@ -929,10 +1075,11 @@ __global__ __launch_bounds__(1024) void batch_owner_kernel(const BatchProblem *_
   while (w < nwork) {
     if (threadIdx.x == 0) item[buf ^ 1u] = atomicAdd(&queue[0], 1u);
     const uint2 pb = work[w];
-    const EngineArgs &a = probs[pb.x].args;
-    double *iterate = const_cast<double *>(a.point_data[0]);
-    const RunIO io{from_iterate ? iterate : a.out, a.out, to_iterate ? iterate : nullptr, nullptr};
-    owner_block<F, SOA>(a, probs[pb.x].hier, io, pb.y, lds);
+    const BatchProblem p = as_global(probs[pb.x]);
+    double *iterate = const_cast<double *>(p.args.point_data[0]);
+    const RunIO io{from_iterate ? iterate : p.args.out, p.args.out, to_iterate ? iterate : nullptr,
+                   nullptr};
+    owner_block<F, SOA>(p.args, p.hier, io, pb.y, lds);
     __syncthreads(); // this item's LDS no longer read; the next index visible
     buf ^= 1u;
     w = item[buf];
@@ -944,6 +1091,25 @@ __global__ __launch_bounds__(1024) void batch_owner_kernel(const BatchProblem *_
       atomicExch(&queue[1], 0u);
     }
   }
+}
+
+// The same on items with gathered sums: one workgroup per item, dealt by the
+// hardware.  As a persistent grid on the queue the kernel needs 92 registers
+// instead of 80, two workgroups per CU instead of three, and each waits at its
+// item's end: 32 meshes of 10^4 to 2 10^5 cells, parts of 512, 127 us a step
+// against 95 (colour loop on the queue: 133).  Items in list order: one
+// contiguous run per XCD, as a single mesh's launch has, measured 100.
+template <class F, bool SOA>
+__global__ __launch_bounds__(512) void batch_owner_gather_kernel(
+    const BatchProblem *__restrict__ probs, const OwnerItem *__restrict__ work, bool from_iterate,
+    bool to_iterate) {
+  extern __shared__ double lds[];
+  const OwnerItem it = work[blockIdx.x];
+  const BatchProblem p = as_global(probs[it.problem]);
+  double *iterate = const_cast<double *>(p.args.point_data[0]);
+  const RunIO io{from_iterate ? iterate : p.args.out, p.args.out, to_iterate ? iterate : nullptr,
+                 nullptr};
+  owner_gather_block<F, SOA>(p.args, p.hier, io, it, lds);
 }
 
 // Batched copies: item i copies count doubles (<= kCopyChunk) src -> dst.
@@ -1677,6 +1843,7 @@ struct fot_loop {
   uint32_t lds_bytes = 0, threads = 0;
   bool staged = false;
   uint32_t gather_rounds = 1;
+  bool may_gather = true; // off for the problems of a batch that cannot all gather
   bool gather = false;   // hierarchical: points gather their increments (eng_gather_kernel)
   bool stage_pd = false; // generic hierarchical: the functor's staged input in LDS
   bool dep_order = false;
@@ -1805,6 +1972,16 @@ struct fot_loop {
   }
 
   // the plan of eng_gather_kernel, when the blocks allow it: sets `gather`
+  // the same for owner_gather_block
+  fot_status build_owner_gather(const std::vector<uint32_t> &blk_cell_off,
+                                const std::vector<uint32_t> &blk_cache_off,
+                                const std::vector<uint32_t> &blk_owned,
+                                const std::vector<uint32_t> &cached,
+                                const std::vector<uint16_t> &loc,
+                                const std::vector<uint8_t> &colour,
+                                const std::vector<uint32_t> &plan_cell);
+  std::vector<OwnerItem> owner_items;
+  uint32_t most_cells = 0, most_owned = 0;
   fot_status build_gather(const std::vector<uint32_t> &blk_cell_off,
                           const std::vector<uint32_t> &blk_cache_off,
                           const std::vector<uint16_t> &loc,
@@ -2015,6 +2192,91 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
     if ((st = upload(plan_cell.data(), plan_cell.size(), &d32)) != FOT_OK) return st;
     hier.cell_ids = d32;
   }
+  lds_bytes = lds;
+  gather = true;
+  return FOT_OK;
+}
+
+fot_status fot_loop::build_owner_gather(
+    const std::vector<uint32_t> &blk_cell_off, const std::vector<uint32_t> &blk_cache_off,
+    const std::vector<uint32_t> &blk_owned, const std::vector<uint32_t> &cached,
+    const std::vector<uint16_t> &loc, const std::vector<uint8_t> &colour,
+    const std::vector<uint32_t> &plan_cell) {
+  const uint32_t md = desc.mesh_dim[0], nb = uint32_t(blk_owned.size());
+  bool takes = false, targets = false;
+  uint32_t lds = 0;
+  for (uint32_t b = 0; b < nb; ++b) {
+    most_cells = std::max(most_cells, blk_cell_off[b + 1] - blk_cell_off[b]);
+    most_owned = std::max(most_owned, blk_owned[b]);
+  }
+  const uint32_t cap = std::max(1u, most_cells);
+  fot_status st = dispatch(&f, desc.soa, [&]<class F, bool SOA>() -> fot_status {
+    takes = kOwnerGathers<F>;
+    targets = kNeedsTargets<F>;
+    if constexpr (kOwnerGathers<F>) lds = owner_gather_lds<F>(cap);
+    return FOT_OK;
+  });
+  const uint32_t most = std::max((most_cells + kOwnerCells - 1) / kOwnerCells,
+                                 (most_owned + kOwnerPoints - 1) / kOwnerPoints);
+  const uint32_t t = std::max<uint32_t>(64, (most + 63) / 64 * 64);
+  if (st != FOT_OK || !takes || t > 512 || md * cap > 0xfffeu || lds > 80u * 1024u) return st;
+  uint64_t owned = 0;
+  for (uint32_t n : blk_owned) owned += n;
+  std::vector<uint16_t> lists(size_t(owned) * 8, uint16_t(md * cap));
+  std::vector<uint32_t> ids(owned), at;
+  std::vector<uint8_t> count;
+  uint32_t longest = 0, o0 = 0;
+  owner_items.resize(nb);
+  for (uint32_t b = 0; b < nb; ++b) {
+    const uint32_t e0 = blk_cell_off[b], ne = blk_cell_off[b + 1] - e0, nw = blk_owned[b];
+    OwnerItem &it = owner_items[b];
+    it = OwnerItem{0, e0, ne, o0, nw, nw ? cached[blk_cache_off[b]] : 0u, 0, 0};
+    for (uint32_t i = 0; i < nw; ++i) {
+      ids[o0 + i] = cached[blk_cache_off[b] + i];
+      if (ids[o0 + i] != it.first + i) it.first = kExclusive;
+    }
+    // by thread colour, then by position, then by slot
+    at.resize(ne);
+    std::iota(at.begin(), at.end(), 0u);
+    std::stable_sort(at.begin(), at.end(),
+                     [&](uint32_t x, uint32_t y) { return colour[e0 + x] < colour[e0 + y]; });
+    count.assign(nw, 0);
+    for (uint32_t i : at)
+      for (uint32_t k = 0; k < md; ++k) {
+        const uint32_t l = loc[size_t(e0 + i) * md + k];
+        if (l >= nw) continue;
+        if (count[l] == 8) return FOT_OK;
+        lists[size_t(o0 + l) * 8 + count[l]++] = uint16_t(k * cap + i);
+        longest = std::max<uint32_t>(longest, count[l]);
+      }
+    if (nw == 0) return FOT_OK;
+    o0 += nw;
+  }
+  if (longest <= 4) {
+    for (size_t i = 0; i < owned; ++i)
+      for (size_t j = 0; j < 4; ++j) lists[4 * i + j] = lists[8 * i + j];
+    lists.resize(4 * owned);
+  }
+  uint32_t *d32 = nullptr;
+  uint16_t *d16 = nullptr;
+  OwnerItem *di = nullptr;
+  if ((st = upload(owner_items.data(), nb, &di)) != FOT_OK) return st;
+  hier.items = di;
+  if ((st = upload(lists.data(), lists.size(), &d16)) != FOT_OK) return st;
+  hier.lists = reinterpret_cast<const uint32_t *>(d16);
+  hier.wide = longest > 4;
+  hier.cap = cap;
+  if ((st = upload(ids.data(), ids.size(), &d32)) != FOT_OK) return st;
+  hier.cached = d32;
+  if (targets) {
+    std::vector<uint32_t> maps(plan_cell.size() * md);
+    for (size_t i = 0; i < plan_cell.size(); ++i)
+      std::memcpy(&maps[i * md], desc.cell_to_node[0] + size_t(plan_cell[i]) * md,
+                  md * sizeof(uint32_t));
+    if ((st = upload(maps.data(), maps.size(), &d32)) != FOT_OK) return st;
+    plan_args.maps[0] = d32;
+  }
+  threads = t;
   lds_bytes = lds;
   gather = true;
   return FOT_OK;
@@ -2422,8 +2684,12 @@ fot_status fot_loop::build_hierarchical() {
   ept = (owner && f.kernel == FOT_KERNEL_RES_CALC && (cfg.flags & FOT_LOOP_TWO_PER_THREAD)) ? 2 : 1;
   threads = std::max<uint32_t>(64, ((max_block + ept - 1) / ept + 63) / 64 * 64);
   if (threads > 1024) return fail(FOT_ERR_UNSUPPORTED, "blocks above 1024 cells");
-  if (!owner && !dep_order && !staged &&
+  if (may_gather && !owner && !dep_order && !staged &&
       (st = build_gather(blk_cell_off, blk_cache_off, loc, plan_cell)) != FOT_OK)
+    return st;
+  if (may_gather && owner &&
+      (st = build_owner_gather(blk_cell_off, blk_cache_off, blk_owned, cached, loc, colour,
+                                        plan_cell)) != FOT_OK)
     return st;
   if (!gather) {
     if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
@@ -2601,6 +2867,13 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
 #undef FOT_OWNER2P
       } else {
         bool done = false;
+        if constexpr (kOwnerGathers<F>) {
+          if (gather) {
+            hipLaunchKernelGGL((eng_owner_gather_kernel<F, SOA>), dim3(nb), dim3(threads),
+                               lds_bytes, s, plan_args, hier, io, nb);
+            done = true;
+          }
+        }
         if constexpr (kSmallBound<F> < 1024) {
           if (threads <= uint32_t(kSmallBound<F>)) {
             hipLaunchKernelGGL((eng_owner_kernel<F, SOA, kSmallBound<F>>), dim3(nb), dim3(threads),
@@ -2677,7 +2950,8 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
 }
 
 static fot_status fot_loop_create_impl(const fot_functor *f, const fot_problem_desc *desc,
-                                      const fot_loop_config *cfg, fot_loop **out) {
+                                      const fot_loop_config *cfg, fot_loop **out,
+                                      bool may_gather = true) {
   if (!f || !desc || !cfg || !out) return fail(FOT_ERR_INVALID_ARGUMENT, "null argument");
   *out = nullptr;
   if (desc->num_mappings == 0 || desc->num_mappings > FOT_MAX_MAPPINGS ||
@@ -2759,6 +3033,7 @@ static fot_status fot_loop_create_impl(const fot_functor *f, const fot_problem_d
   L->base.out = desc->point_data_out;
   L->base.num_cells = desc->num_cells;
   L->base.cell_stride = desc->num_cells;
+  L->may_gather = may_gather;
   L->stats.strategy = cfg->strategy;
   L->stats.block_size = cfg->block_size;
   fot_status st;
@@ -2928,6 +3203,7 @@ struct fot_batch {
   std::vector<void *> owned;
   BatchProblem *probs = nullptr;
   uint2 *work = nullptr;
+  OwnerItem *items = nullptr; // the work items when every problem's points gather
   uint32_t nwork = 0;
   uint32_t *queue = nullptr;
   CopyItem *copy_in = nullptr, *copy_back = nullptr; // out <- in, in <- out
@@ -2956,6 +3232,14 @@ struct fot_batch {
   fot_status launch_step(hipStream_t s, bool from_iterate = false, bool to_iterate = false) {
     if (nwork == 0) return FOT_OK;
     return dispatch(&f, soa, [&]<class F, bool SOA>() -> fot_status {
+      if constexpr (kOwnerGathers<F>) {
+        if (items) {
+          hipLaunchKernelGGL((batch_owner_gather_kernel<F, SOA>), dim3(grid), dim3(threads),
+                             lds_bytes, s, probs, items, from_iterate, to_iterate);
+          FOT_HIP(hipGetLastError());
+          return FOT_OK;
+        }
+      }
       hipLaunchKernelGGL((batch_owner_kernel<F, SOA>), dim3(grid), dim3(threads), lds_bytes, s,
                          probs, work, nwork, queue, from_iterate, to_iterate);
       FOT_HIP(hipGetLastError());
@@ -2984,6 +3268,7 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
   fot_status st;
   std::vector<BatchProblem> host(num_problems);
   std::vector<CopyItem> cin, cback;
+  bool gather = true;
   for (uint32_t i = 0; i < num_problems; ++i) {
     if (descs[i].soa != B->soa)
       return fail(FOT_ERR_INVALID_ARGUMENT, "problem %u: every problem needs the same layout", i);
@@ -2992,8 +3277,18 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
     c.flags = (c.flags & FOT_LOOP_POINT_PARTITION) | FOT_LOOP_OWNER_COMPUTE;
     c.use_graph = 0;
     fot_loop *l = nullptr;
-    if ((st = fot_loop_create(f, &descs[i], &c, &l)) != FOT_OK) return st;
+    if ((st = fot_loop_create_impl(f, &descs[i], &c, &l, gather)) != FOT_OK) return st;
     B->loops.push_back(l);
+    if (gather && !l->gather && l->colour_blk_off.back() > 0) {
+      // one kernel runs every problem: plan them all for the colour loop
+      gather = false;
+      for (fot_loop *p : B->loops) delete p;
+      B->loops.clear();
+      i = 0xffffffffu;
+    }
+  }
+  for (uint32_t i = 0; i < num_problems; ++i) {
+    const fot_loop *l = B->loops[i];
     host[i].args = l->plan_args;
     host[i].hier = l->hier;
     B->threads = std::max(B->threads, l->threads);
@@ -3022,10 +3317,17 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
     return descs[a].num_cells > descs[b].num_cells;
   });
   std::vector<uint2> work;
+  std::vector<OwnerItem> items;
   for (uint32_t i : order) {
     const uint32_t nb = B->loops[i]->colour_blk_off.back();
     for (uint32_t b = 0; b < nb; ++b) work.push_back(make_uint2(i, b));
+    if (!gather) continue;
+    for (OwnerItem it : B->loops[i]->owner_items) {
+      it.problem = i;
+      items.push_back(it);
+    }
   }
+  if (gather && !items.empty() && (st = B->upload(items, &B->items)) != FOT_OK) return st;
   B->nwork = uint32_t(work.size());
   B->ncopy = uint32_t(cin.size());
   if ((st = B->upload(host, &B->probs)) != FOT_OK) return st;
@@ -3035,18 +3337,23 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
   if ((st = B->upload(std::vector<uint32_t>{0u, 0u}, &B->queue)) != FOT_OK) return st;
   if (B->lds_bytes > 160u * 1024u)
     return fail(FOT_ERR_UNSUPPORTED, "batch needs %u B of LDS", B->lds_bytes);
-  // persistent grid: as many workgroups as fit on the device at once
-  int dev = 0, cus = 0, per_cu = 0;
-  FOT_HIP(hipGetDevice(&dev));
-  FOT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  st = dispatch(f, B->soa, [&]<class F, bool SOA>() -> fot_status {
-    FOT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void *>(&batch_owner_kernel<F, SOA>), int(B->threads),
-        size_t(B->lds_bytes)));
-    return FOT_OK;
-  });
-  if (st != FOT_OK) return st;
-  B->grid = std::max<uint32_t>(1, std::min<uint32_t>(B->nwork, uint32_t(std::max(1, per_cu) * cus)));
+  if (B->items) {
+    B->grid = B->nwork;
+  } else {
+    // persistent grid: as many workgroups as fit on the device at once
+    int dev = 0, cus = 0, per_cu = 0;
+    FOT_HIP(hipGetDevice(&dev));
+    FOT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    st = dispatch(f, B->soa, [&]<class F, bool SOA>() -> fot_status {
+      FOT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &per_cu, reinterpret_cast<const void *>(&batch_owner_kernel<F, SOA>), int(B->threads),
+          size_t(B->lds_bytes)));
+      return FOT_OK;
+    });
+    if (st != FOT_OK) return st;
+    B->grid =
+        std::max<uint32_t>(1, std::min<uint32_t>(B->nwork, uint32_t(std::max(1, per_cu) * cus)));
+  }
   FOT_HIP(hipDeviceSynchronize());
   if (use_graph && (B->nwork > 0 || B->jacobi)) {
     // one timestep: the batched increments, then in <- out for every problem

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from cuda_fot_amd import Problem, capi, meshgen, plan
+from cuda_fot_amd import Problem, capi, gpu_batch, meshgen, plan
 from helpers import (airfoil_problem, assert_bitwise, assert_close_scaled, hex_problem,
                      mine_problem, oracle_of)
 
@@ -306,6 +306,37 @@ def test_gathered_sums_at_their_limits(gpu, kind, soa):
             p.gpu_loop(capi.functor(capi.KERNEL_MINE, md, 4, 4), capi.STRATEGY_HIERARCHICAL, 2,
                        flags=flags)
             assert_bitwise(p.point_data[0], ref, f"{kind} flags {flags}")
+
+
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("kind", ["hubs4", "hubs8", "hubs9", "twice"])
+def test_owner_gathered_sums_at_their_limits(gpu, kind, soa):
+    """The owner blocks' gathered sums on the same meshes, single and as a
+    batch with a mesh that gathers, with zeros of either sign among the values,
+    points no cell names, and parts whose ids are not consecutive."""
+    maps, n, md, bs = _gather_mesh(kind)
+    n += 70  # parts of points alone
+    f = capi.functor(capi.KERNEL_MINE, md, 4, 4)
+
+    def problem():
+        pd = meshgen.uniform(n * 4, 1).reshape(n, 4)
+        pd[::3] = -0.0
+        w = meshgen.uniform(maps.shape[0] * 4, 2, -1.0, 1.0).reshape(4, -1)
+        return Problem([maps], [n], [pd.T.copy() if soa else pd], [w], bs, soa)
+
+    scattered = (np.arange(n) % (-(-n // bs))).astype(np.uint32)
+    for part in (None, scattered):
+        ref = _owner_replay(problem(), O.MINE2, bs, None, 2, part)
+        p = problem()
+        p.point_partition = part
+        p.gpu_loop(f, capi.STRATEGY_HIERARCHICAL, 2, flags=OWN)
+        assert_bitwise(p.point_data[0], ref, kind)
+        both = [problem(), mine_problem(N=20, M=9, seed=3, soa=soa, block_size=64)]
+        both[0].point_partition = part
+        other = _owner_replay(copy.deepcopy(both[1]), O.MINE2, 64, None, 2)
+        gpu_batch(both, f, 2)
+        assert_bitwise(both[0].point_data[0], ref, f"{kind} in a batch")
+        assert_bitwise(both[1].point_data[0], other, f"beside {kind} in a batch")
 
 
 @pytest.mark.parametrize("iters", [1, 2, 3])
