@@ -809,6 +809,113 @@ __global__ __launch_bounds__(1024) void res_calc_hier_staged_kernel(EngineArgs a
   publish<DEP>(dd, b, gen);
 }
 
+// The same with gathered sums (see eng_gather_kernel), for launches per block
+// colour and two-phase ones: an edge stores its flux f, and a point's list names
+// the fluxes it adds or, as the edge's second cell, subtracts (place | 0x8000;
+// its increment is -f, and v + (-f) is v - f).
+template <bool SOA, int R>
+__global__ __launch_bounds__(1024) void res_calc_hier_gather_kernel(EngineArgs a, HierDev h,
+                                                                    RunIO io, uint32_t blk_begin,
+                                                                    uint32_t nbc) {
+  extern __shared__ double lds[];
+  const uint4 rec = h.rec[blk_begin + xcd_block(blockIdx.x, nbc)];
+  const uint32_t tid = threadIdx.x, T = blockDim.x, e0 = rec.x, ne = rec.y, c0 = rec.z, m = rec.w;
+  const double *x = a.point_data[1], *q = a.point_data[2], *adt = a.point_data[3];
+  const uint32_t np = a.num_points[0], nq = a.num_points[2], nx = a.num_points[1];
+  const uint32_t pos = e0 + min(tid, ne - 1);
+  uint32_t g[R], slot[R];
+  uint4 list[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) g[r] = h.cached[c0 + min(tid + r * T, m - 1)];
+  const uint2 nn = reinterpret_cast<const uint2 *>(a.maps[1])[pos];
+  const uint32_t lv = reinterpret_cast<const uint32_t *>(h.loc)[pos];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t entry = c0 + min(tid + r * T, m - 1);
+    if (h.wide) {
+      list[r] = reinterpret_cast<const uint4 *>(h.lists)[entry];
+    } else {
+      const uint2 w = reinterpret_cast<const uint2 *>(h.lists)[entry];
+      list[r] = make_uint4(w.x, w.y, 0u, 0u);
+    }
+    slot[r] = h.wslot ? h.wslot[entry] : kExclusive;
+  }
+  double qv[R][4], av[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) qv[r][d] = q[pidx<SOA>(nq, g[r], 4, d)];
+    av[r] = adt[g[r]];
+  }
+  double x1[2], x2[2];
+#pragma unroll
+  for (uint32_t d = 0; d < 2; ++d)
+    x1[d] = x[pidx<SOA>(nx, nn.x, 2, d)], x2[d] = x[pidx<SOA>(nx, nn.y, 2, d)];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t i = tid + r * T;
+    if (i < m) {
+#pragma unroll
+      for (uint32_t d = 0; d < 4; ++d) lds[d * m + i] = qv[r][d];
+      lds[4 * m + i] = av[r];
+    }
+  }
+  __syncthreads();
+  double f[4], f2[4];
+  if (tid < ne) {
+    const uint32_t l0 = lv & 0xffffu, l1 = lv >> 16;
+    double q1[4], q2[4];
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) q1[d] = lds[d * m + l0], q2[d] = lds[d * m + l1];
+    const double a1 = lds[4 * m + l0], a2 = lds[4 * m + l1];
+    res_calc_user(x1, x2, q1, q2, &a1, &a2, f, f2, 1, 1);
+  }
+  __syncthreads(); // the fluxes take the staged values' place
+  const uint32_t stride = T + 1; // + a zero for empty places
+  if (tid < ne) {
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) lds[d * stride + tid] = f[d];
+  }
+  if (tid < 4) lds[tid * stride + T] = 0.0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (tid + r * T >= m) continue;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add4 = [&](uint32_t lo, uint32_t hi) {
+      const uint32_t at[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const bool minus = at[j] & 0x8000u;
+#pragma unroll
+        for (uint32_t d = 0; d < 4; ++d) {
+          const double w = lds[d * stride + (at[j] & 0x7fffu)];
+          v[d] += minus ? -w : w;
+        }
+      }
+    };
+    add4(list[r].x, list[r].y);
+    if (h.wide) add4(list[r].z, list[r].w);
+    if (slot[r] == kExclusive) {
+      double o[4];
+#pragma unroll
+      for (uint32_t d = 0; d < 4; ++d) o[d] = io.base[pidx<SOA>(np, g[r], 4, d)];
+#pragma unroll
+      for (uint32_t d = 0; d < 4; ++d) {
+        v[d] = o[d] + v[d];
+        io.out[pidx<SOA>(np, g[r], 4, d)] = v[d];
+      }
+      if (io.also) {
+#pragma unroll
+        for (uint32_t d = 0; d < 4; ++d) io.also[pidx<SOA>(np, g[r], 4, d)] = v[d];
+      }
+    } else {
+#pragma unroll
+      for (uint32_t d = 0; d < 4; ++d) h.partial[size_t(slot[r]) * 4 + d] = v[d];
+    }
+  }
+}
+
 // ---- owner-compute launches -----------------------------------------------
 // One launch over all blocks.  A block's LDS cache holds the current values
 // of its owned points, loaded while its inputs are staged; the increments of
@@ -2138,10 +2245,25 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
   });
   if (st != FOT_OK) return st;
   if (stage_pd && !stages) return FOT_OK; // eng_hier_kernel stages the others' input
+  // res_calc_hier_gather_kernel, where the plan's blocks do not fill the chip
+  // for one round and their latency is what counts (colour loop / this, a
+  // step: 64x32 8.9 / 7.2 us, 200x150 10.0 / 7.6, blocks of 512; 701x463,
+  // blocks of 1024, 20.6 / 18.1); beyond that its registers and LDS traffic
+  // cost as much as they save (701x463, blocks of 512, SOA 25.0 / 25.0;
+  // 2400x1200 AOS 154.1 / 154.4, SOA 157 / 169)
+  if (staged && nb >= 1024) return FOT_OK;
+  if (staged) {
+    stages = true, targets = false;
+    lds = 0;
+    for (uint32_t b = 0; b < nb; ++b)
+      lds = std::max(lds, 8u * std::max(5u * (blk_cache_off[b + 1] - blk_cache_off[b]),
+                                        4u * (threads + 1)));
+  }
   if (lds > 160u * 1024u || md * threads > 0xfffeu) return FOT_OK;
   // A point's increments in the order of the plan's cells, which are sorted by
   // thread colour, then by the cell's slots.
-  const uint16_t none = uint16_t(md * threads);
+  const uint16_t none = uint16_t(staged ? threads : md * threads);
+  const uint32_t slot_step = staged ? 0x8000u : threads;
   std::vector<uint16_t> lists(size_t(blk_cache_off[nb]) * 8, none);
   std::vector<uint8_t> count;
   std::vector<uint4> rec(nb);
@@ -2156,7 +2278,7 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
       for (uint32_t k = 0; k < md; ++k) {
         const uint32_t l = loc[size_t(e0 + i) * md + k];
         if (count[l] == 8) return FOT_OK;
-        lists[size_t(c0 + l) * 8 + count[l]++] = uint16_t(k * threads + i);
+        lists[size_t(c0 + l) * 8 + count[l]++] = uint16_t(k * slot_step + i);
         longest = std::max<uint32_t>(longest, count[l]);
       }
   }
@@ -2238,8 +2360,9 @@ fot_status fot_loop::build_owner_gather(
     // by thread colour, then by position, then by slot
     at.resize(ne);
     std::iota(at.begin(), at.end(), 0u);
-    std::stable_sort(at.begin(), at.end(),
-                     [&](uint32_t x, uint32_t y) { return colour[e0 + x] < colour[e0 + y]; });
+    if (!std::is_sorted(colour.begin() + e0, colour.begin() + e0 + ne))
+      std::stable_sort(at.begin(), at.end(),
+                       [&](uint32_t x, uint32_t y) { return colour[e0 + x] < colour[e0 + y]; });
     count.assign(nw, 0);
     for (uint32_t i : at)
       for (uint32_t k = 0; k < md; ++k) {
@@ -2266,8 +2389,11 @@ fot_status fot_loop::build_owner_gather(
   hier.lists = reinterpret_cast<const uint32_t *>(d16);
   hier.wide = longest > 4;
   hier.cap = cap;
-  if ((st = upload(ids.data(), ids.size(), &d32)) != FOT_OK) return st;
-  hier.cached = d32;
+  if (std::any_of(owner_items.begin(), owner_items.end(),
+                  [](const OwnerItem &it) { return it.first == kExclusive; })) {
+    if ((st = upload(ids.data(), ids.size(), &d32)) != FOT_OK) return st;
+    hier.cached = d32;
+  }
   if (targets) {
     std::vector<uint32_t> maps(plan_cell.size() * md);
     for (size_t i = 0; i < plan_cell.size(); ++i)
@@ -2684,7 +2810,7 @@ fot_status fot_loop::build_hierarchical() {
   ept = (owner && f.kernel == FOT_KERNEL_RES_CALC && (cfg.flags & FOT_LOOP_TWO_PER_THREAD)) ? 2 : 1;
   threads = std::max<uint32_t>(64, ((max_block + ept - 1) / ept + 63) / 64 * 64);
   if (threads > 1024) return fail(FOT_ERR_UNSUPPORTED, "blocks above 1024 cells");
-  if (may_gather && !owner && !dep_order && !staged &&
+  if (may_gather && !owner && !dep_order &&
       (st = build_gather(blk_cell_off, blk_cache_off, loc, plan_cell)) != FOT_OK)
     return st;
   if (may_gather && owner &&
@@ -2904,13 +3030,18 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
       const uint32_t nb = colour_blk_off.back();
       bool done = false;
       if constexpr (std::is_same<F, ResCalcF>::value) {
-        if (staged) {
+        if (staged && gather) {
+          hipLaunchKernelGGL((gather_rounds == 1 ? res_calc_hier_gather_kernel<SOA, 1>
+                                                 : res_calc_hier_gather_kernel<SOA, 2>),
+                             dim3(nb), dim3(threads), lds_bytes, s, plan_args, hier, io, 0u, nb);
+          done = true;
+        } else if (staged) {
           hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 2>), dim3(nb), dim3(threads),
                              lds_bytes, s, plan_args, hier, dep, 0u, nb);
           done = true;
         }
       }
-      if (gather) {
+      if (gather && !done) {
         if (gather_rounds == 1)
           launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, io, 0u, nb, nontemporal);
         else
@@ -2927,6 +3058,13 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
         const uint32_t b0 = colour_blk_off[c], nbc = colour_blk_off[c + 1] - b0;
         if (nbc == 0) continue;
         if constexpr (std::is_same<F, ResCalcF>::value) {
+          if (staged && gather) {
+            hipLaunchKernelGGL((gather_rounds == 1 ? res_calc_hier_gather_kernel<SOA, 1>
+                                                 : res_calc_hier_gather_kernel<SOA, 2>),
+                               dim3(nbc), dim3(threads), lds_bytes, s, plan_args, hier, io, b0,
+                               nbc);
+            continue;
+          }
           if (staged) {
             hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 0>), dim3(nbc),
                                dim3(threads), lds_bytes, s, plan_args, hier, dep, b0, nbc);
