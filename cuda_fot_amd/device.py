@@ -126,7 +126,7 @@ def make_desc(maps, num_points, point_data, out, cell_data=(), soa=False):
 
 
 class Batch:
-    """Many problems of one functor run by one persistent launch per step
+    """Many problems of one functor run by one launch per step
     (fot_batch).  Each problem: dict(maps, num_points, point_data, out,
     cell_data, soa, block_size, point_partition=None) with device arrays."""
 

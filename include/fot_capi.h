@@ -586,8 +586,9 @@ fot_status fot_loop_stats_get(const fot_loop *loop, fot_loop_stats *stats);
 /* ------------------------------------------------------------------ */
 /* Batched loops (no reference counterpart): many problems of one        */
 /* functor, each planned as an owner-compute hierarchical loop with its  */
-/* own config, run together by ONE persistent launch per step whose      */
-/* workgroups take (problem, block) items from a device work queue.      */
+/* own config, run together by ONE launch per step over (problem, block) */
+/* items: a workgroup per item, or (functors whose points do not gather) */
+/* a persistent grid that takes them from a device work queue.           */
 /* ------------------------------------------------------------------ */
 typedef struct fot_batch fot_batch;
 /* descs/cfgs: one per problem (same functor and layout).  Each cfg's
