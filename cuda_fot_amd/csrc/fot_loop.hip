@@ -86,6 +86,13 @@ struct RunIO {
   double *cells; // the caller's array for the functor's cell output, or null
                  // (then the plan-order copy)
 };
+// A plain step's argument in its place: the owner kernels of a step neither
+// load nor test what only a run needs.  With one kernel for both, a step of a
+// few blocks paid for it (64x32 airfoil, owner compute: 4.11 us without, 4.38
+// with, 4.17-4.26 as two kernels; a full chip's step is the same).
+struct StepIO {};
+FOT_DEV RunIO run_io(const EngineArgs &a, StepIO) { return {a.out, a.out, nullptr, nullptr}; }
+FOT_DEV RunIO run_io(const EngineArgs &, const RunIO &run) { return run; }
 
 // Two-phase writeback of a block's cache entry i (point g, values v): added
 // in place when this block alone touches g, else stored in its partial slot
@@ -1117,18 +1124,18 @@ __device__ __forceinline__ void owner_gather_block(const EngineArgs &a, const Hi
   }
 }
 
-template <class F, bool SOA>
-__global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, HierDev h, RunIO io,
-                                                               uint32_t nb) {
+template <class F, bool SOA, class IO>
+__global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, HierDev h,
+                                                               uint32_t nb, IO run) {
   extern __shared__ double lds[];
-  owner_gather_block<F, SOA>(a, h, io, h.items[xcd_block(blockIdx.x, nb)], lds);
+  owner_gather_block<F, SOA>(a, h, run_io(a, run), h.items[xcd_block(blockIdx.x, nb)], lds);
 }
 
-template <class F, bool SOA, int LB = 1024>
-__global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, RunIO io,
-                                                       uint32_t nb) {
+template <class F, bool SOA, class IO, int LB = 1024>
+__global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, uint32_t nb,
+                                                       IO run) {
   extern __shared__ double lds[];
-  owner_block<F, SOA>(a, h, io, xcd_block(blockIdx.x, nb), lds);
+  owner_block<F, SOA>(a, h, run_io(a, run), xcd_block(blockIdx.x, nb), lds);
 }
 
 // One problem of a batch: its engine arguments and owner-compute plan.
@@ -1684,14 +1691,15 @@ FOT_DEV void owner3_body(double *lds, Owner3Data<EPT, KS, KO> &d, const Owner3Id
   }
 }
 
-template <bool SOA, int EPT, int KS, int LW, int KO, bool PRE>
+template <bool SOA, int EPT, int KS, int LW, int KO, bool PRE, class IO>
 __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
                                                                const OwnerMeta *__restrict__ meta,
                                                                const uint32_t *__restrict__ cached,
                                                                const uint32_t *__restrict__ packed,
                                                                const uint32_t *__restrict__ plist,
-                                                               RunIO io, uint32_t nb) {
+                                                               uint32_t nb, IO run) {
   extern __shared__ double lds[];
+  const RunIO io = run_io(a, run);
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
@@ -1704,12 +1712,13 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
 
 // The same with the owned res loaded and stored nontemporally (edge lists
 // built in LDS, no per-cell terms): the same bits.
-template <bool SOA, int EPT, int KS, int KO>
+template <bool SOA, int EPT, int KS, int KO, class IO>
 __global__ __launch_bounds__(1024) void res_calc_owner3_stream_kernel(
     EngineArgs a, const OwnerMeta *__restrict__ meta, const uint32_t *__restrict__ cached,
-    const uint32_t *__restrict__ packed, const uint32_t *__restrict__ plist, RunIO io,
-    uint32_t nb) {
+    const uint32_t *__restrict__ packed, const uint32_t *__restrict__ plist, uint32_t nb,
+    IO run) {
   extern __shared__ double lds[];
+  const RunIO io = run_io(a, run);
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
@@ -1726,14 +1735,15 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_stream_kernel(
 // chunk.  The next block's record and ids load while the current block's
 // body runs, so after its first block a workgroup waits for one round trip
 // per block (the data), not two.  Same per-block arithmetic: the same bits.
-template <bool SOA, int EPT, int KS, int LW, int KO, bool PRE>
+template <bool SOA, int EPT, int KS, int LW, int KO, bool PRE, class IO>
 __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
                                                                const OwnerMeta *__restrict__ meta,
                                                                const uint32_t *__restrict__ cached,
                                                                const uint32_t *__restrict__ packed,
                                                                const uint32_t *__restrict__ plist,
-                                                               RunIO io, uint32_t nb) {
+                                                               uint32_t nb, IO run) {
   extern __shared__ double lds[];
+  const RunIO io = run_io(a, run);
   const uint32_t tid = threadIdx.x, bd = blockDim.x, G = gridDim.x;
   uint32_t j = blockIdx.x;
   if (j >= nb) return;
@@ -1760,48 +1770,48 @@ __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
 
 // the gather kernel instantiation for a plan: one block per workgroup or
 // persistent, edges per thread, staging rounds, list words, owned rounds
-template <bool SOA, int E, int K, int W, int O>
+template <bool SOA, int E, int K, int W, int O, class IO>
 const void *owner3_pick(bool persistent, bool pre) {
   if (pre)
     return persistent
-               ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, true>)
-               : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, true>);
+               ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, true, IO>)
+               : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, true, IO>);
   return persistent
-             ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, false>)
-             : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, false>);
+             ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, false, IO>)
+             : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, false, IO>);
 }
-template <bool SOA, int E, int K>
+template <bool SOA, int E, int K, class IO>
 const void *owner3_pick_w(bool persistent, bool pre, uint32_t lw, bool ko1, bool nt) {
   if (lw == 0 && nt && !persistent && !pre)
-    return ko1 ? reinterpret_cast<const void *>(&res_calc_owner3_stream_kernel<SOA, E, K, 1>)
-               : reinterpret_cast<const void *>(&res_calc_owner3_stream_kernel<SOA, E, K, K>);
+    return ko1 ? reinterpret_cast<const void *>(&res_calc_owner3_stream_kernel<SOA, E, K, 1, IO>)
+               : reinterpret_cast<const void *>(&res_calc_owner3_stream_kernel<SOA, E, K, K, IO>);
   if (lw == 0)
-    return ko1 ? owner3_pick<SOA, E, K, 0, 1>(persistent, pre)
-               : owner3_pick<SOA, E, K, 0, K>(persistent, pre);
+    return ko1 ? owner3_pick<SOA, E, K, 0, 1, IO>(persistent, pre)
+               : owner3_pick<SOA, E, K, 0, K, IO>(persistent, pre);
   if (lw == 2)
-    return ko1 ? owner3_pick<SOA, E, K, 2, 1>(persistent, pre)
-               : owner3_pick<SOA, E, K, 2, K>(persistent, pre);
-  return ko1 ? owner3_pick<SOA, E, K, 4, 1>(persistent, pre)
-             : owner3_pick<SOA, E, K, 4, K>(persistent, pre);
+    return ko1 ? owner3_pick<SOA, E, K, 2, 1, IO>(persistent, pre)
+               : owner3_pick<SOA, E, K, 2, K, IO>(persistent, pre);
+  return ko1 ? owner3_pick<SOA, E, K, 4, 1, IO>(persistent, pre)
+             : owner3_pick<SOA, E, K, 4, K, IO>(persistent, pre);
 }
-template <bool SOA, int E>
+template <bool SOA, int E, class IO>
 const void *owner3_pick_k(bool persistent, bool pre, uint32_t ks, uint32_t lw, bool ko1,
                           bool nt) {
   switch (ks) {
-  case 1: return owner3_pick_w<SOA, E, 1>(persistent, pre, lw, ko1, nt);
-  case 2: return owner3_pick_w<SOA, E, 2>(persistent, pre, lw, ko1, nt);
-  case 3: return owner3_pick_w<SOA, E, 3>(persistent, pre, lw, ko1, nt);
-  default: return owner3_pick_w<SOA, E, 4>(persistent, pre, lw, ko1, nt);
+  case 1: return owner3_pick_w<SOA, E, 1, IO>(persistent, pre, lw, ko1, nt);
+  case 2: return owner3_pick_w<SOA, E, 2, IO>(persistent, pre, lw, ko1, nt);
+  case 3: return owner3_pick_w<SOA, E, 3, IO>(persistent, pre, lw, ko1, nt);
+  default: return owner3_pick_w<SOA, E, 4, IO>(persistent, pre, lw, ko1, nt);
   }
 }
 // nt: the streaming-output instantiation, which exists for the default form
 // only (one block per workgroup, lists in LDS, no per-cell terms); the other
 // forms ignore it
-template <bool SOA>
+template <bool SOA, class IO>
 const void *owner3_pick_kernel(bool persistent, bool pre, uint32_t ept, uint32_t ks, uint32_t lw,
                                bool ko1, bool nt) {
-  return ept == 2 ? owner3_pick_k<SOA, 2>(persistent, pre, ks, lw, ko1, nt)
-                  : owner3_pick_k<SOA, 1>(persistent, pre, ks, lw, ko1, nt);
+  return ept == 2 ? owner3_pick_k<SOA, 2, IO>(persistent, pre, ks, lw, ko1, nt)
+                  : owner3_pick_k<SOA, 1, IO>(persistent, pre, ks, lw, ko1, nt);
 }
 
 // dst[d * n_dst + i] = src[d * n_src + idx[i]] (SOA gather of cell data)
@@ -1888,6 +1898,26 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
                      lds, s, a, h, dd, b0, nbc);
 }
 
+// Launches eng_owner_gather_kernel or eng_owner_kernel; IO: StepIO or RunIO.
+template <class F, bool SOA, class IO>
+void launch_owner(bool gather, uint32_t nb, uint32_t threads, uint32_t lds, hipStream_t s,
+                  const EngineArgs &a, const HierDev &h, const IO &io) {
+  constexpr int SB = kSmallBound<F>;
+  if constexpr (kOwnerGathers<F>) {
+    if (gather) {
+      hipLaunchKernelGGL((eng_owner_gather_kernel<F, SOA, IO>), dim3(nb), dim3(threads), lds, s, a,
+                         h, nb, io);
+      return;
+    }
+  }
+  if (threads <= uint32_t(SB))
+    hipLaunchKernelGGL((eng_owner_kernel<F, SOA, IO, SB>), dim3(nb), dim3(threads), lds, s, a, h,
+                       nb, io);
+  else
+    hipLaunchKernelGGL((eng_owner_kernel<F, SOA, IO>), dim3(nb), dim3(threads), lds, s, a, h, nb,
+                       io);
+}
+
 // Launches eng_gather_kernel<F, SOA, R>.
 template <class F, bool SOA, int R>
 void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
@@ -1970,7 +2000,9 @@ struct fot_loop {
   bool lists_in_lds = false;     // owner gather: the kernel builds the lists in LDS
   uint32_t stage_per_thread = 1; // owner res_calc: staged points per thread
   bool owned_first_round = false; // owner res_calc: every block owns <= threads cells
-  const void *owner3_fn = nullptr; // owner gather: the kernel instantiation to launch
+  // owner gather: the kernel instantiations to launch for a plain step and for
+  // the first and last step of a run
+  const void *owner3_fn = nullptr, *owner3_run_fn = nullptr;
   // nontemporal hints on read-once data: owner res_calc gather, the owned
   // res; two-phase, the streaming functors' cell data
   bool nontemporal = false;
@@ -2866,12 +2898,14 @@ fot_status fot_loop::build_hierarchical() {
     const bool persistent = (cfg.flags & FOT_LOOP_PERSISTENT) != 0;
     const uint32_t lw = lists_in_lds ? 0u : list_words;
     nontemporal = want_nt && lw == 0 && !persistent && !point_terms;
-    owner3_fn = desc.soa ? owner3_pick_kernel<true>(persistent, point_terms, ept,
-                                                    stage_per_thread, lw, owned_first_round,
-                                                    nontemporal)
-                         : owner3_pick_kernel<false>(persistent, point_terms, ept,
-                                                     stage_per_thread, lw, owned_first_round,
-                                                     nontemporal);
+    auto pick = [&](auto fn) {
+      return fn(persistent, point_terms, ept, stage_per_thread, lw, owned_first_round,
+                nontemporal);
+    };
+    owner3_fn = pick(desc.soa ? owner3_pick_kernel<true, StepIO>
+                              : owner3_pick_kernel<false, StepIO>);
+    owner3_run_fn = pick(desc.soa ? owner3_pick_kernel<true, RunIO>
+                                  : owner3_pick_kernel<false, RunIO>);
     if (persistent && nb_total) {
       // as many workgroups as are resident at once, a multiple of the 8 XCDs
       int dev = 0, cus = 0, per_cu = 0;
@@ -2977,10 +3011,10 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
           const OwnerMeta *om = owner_meta;
           const uint32_t *pc = hier.cached, *pp = hier.packed, *pl = owner_plist;
           uint32_t nbv = nb;
-          RunIO iov = io;
-          void *kargs[] = {&pa, &om, &pc, &pp, &pl, &iov, &nbv};
-          FOT_HIP(hipLaunchKernel(owner3_fn, dim3(launch_grid), dim3(threads), kargs,
-                                  size_t(lds_bytes), s));
+          RunIO iov = io; // (a StepIO takes its first byte)
+          void *kargs[] = {&pa, &om, &pc, &pp, &pl, &nbv, &iov};
+          FOT_HIP(hipLaunchKernel(run ? owner3_run_fn : owner3_fn, dim3(launch_grid),
+                                  dim3(threads), kargs, size_t(lds_bytes), s));
         } else if (ept == 2) {
           if (stage_x) FOT_OWNER2_K(2, true)
           else FOT_OWNER2_K(2, false)
@@ -2992,24 +3026,8 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
 #undef FOT_OWNER2
 #undef FOT_OWNER2P
       } else {
-        bool done = false;
-        if constexpr (kOwnerGathers<F>) {
-          if (gather) {
-            hipLaunchKernelGGL((eng_owner_gather_kernel<F, SOA>), dim3(nb), dim3(threads),
-                               lds_bytes, s, plan_args, hier, io, nb);
-            done = true;
-          }
-        }
-        if constexpr (kSmallBound<F> < 1024) {
-          if (threads <= uint32_t(kSmallBound<F>)) {
-            hipLaunchKernelGGL((eng_owner_kernel<F, SOA, kSmallBound<F>>), dim3(nb), dim3(threads),
-                               lds_bytes, s, plan_args, hier, io, nb);
-            done = true;
-          }
-        }
-        if (!done)
-          hipLaunchKernelGGL((eng_owner_kernel<F, SOA>), dim3(nb), dim3(threads), lds_bytes, s,
-                             plan_args, hier, io, nb);
+        if (run) launch_owner<F, SOA>(gather, nb, threads, lds_bytes, s, plan_args, hier, io);
+        else launch_owner<F, SOA>(gather, nb, threads, lds_bytes, s, plan_args, hier, StepIO{});
       }
     } else if (dep_order) {
       // one launch over every plan block
@@ -3286,7 +3304,7 @@ static fot_status fot_loop_run_impl(fot_loop *loop, uint32_t iters, void *stream
       if (jacobi) io.out = in, io.also = last ? d.point_data_out : nullptr;
       if (last && slot >= 0 && loop->hier.cell_ids)
         io.cells = const_cast<double *>(d.cell_data[slot]);
-      if ((st = loop->enqueue(hs, &io)) != FOT_OK) return st;
+      if ((st = loop->enqueue(hs, it == 0 || last || jacobi ? &io : nullptr)) != FOT_OK) return st;
     }
     if (!loop->hier.cell_ids && (st = loop->scatter_cell_outputs(hs)) != FOT_OK) return st;
     FOT_HIP(hipStreamSynchronize(hs));
