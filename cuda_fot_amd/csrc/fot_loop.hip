@@ -3262,17 +3262,20 @@ bool fot_loop::fuses_run() const {
   if (!(two_phase && gather) &&
       !(owner && !jacobi && (f.kernel != FOT_KERNEL_RES_CALC || owner_gather)))
     return false;
-  // and the iterate is nobody else's: not the output, no other input
-  const double *in = desc.point_data[0];
+  // and the iterate, the output and the cell output are nobody else's: the
+  // copies come before anything is read and the cell output after everything
+  // is written, which no longer holds once they are part of a step
   const uint64_t n = uint64_t(desc.num_points[0]) * desc.point_dim[0];
-  for (uint32_t k = 1; k < desc.num_mappings; ++k)
-    if (overlaps(in, n, desc.point_data[k], uint64_t(desc.num_points[k]) * desc.point_dim[k]))
-      return false;
+  const double *in = desc.point_data[0], *out = base.out;
   const int slot = cell_output_slot(f);
-  if (slot >= 0 && overlaps(in, n, desc.cell_data[slot],
-                            uint64_t(desc.num_cells) * desc.cell_dim[slot]))
-    return false;
-  return !overlaps(in, n, base.out, n);
+  const double *cells = slot >= 0 ? desc.cell_data[slot] : nullptr;
+  const uint64_t nc = slot >= 0 ? uint64_t(desc.num_cells) * desc.cell_dim[slot] : 0;
+  for (uint32_t k = 1; k < desc.num_mappings; ++k) {
+    const double *q = desc.point_data[k];
+    const uint64_t m = uint64_t(desc.num_points[k]) * desc.point_dim[k];
+    if (overlaps(in, n, q, m) || overlaps(out, n, q, m) || overlaps(cells, nc, q, m)) return false;
+  }
+  return !overlaps(in, n, out, n) && !overlaps(in, n, cells, nc) && !overlaps(out, n, cells, nc);
 }
 
 bool fot_loop::keeps_off(const double *p, uint64_t n) const {
@@ -3460,11 +3463,11 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
   B->fused = !use_graph;
   for (uint32_t i = 0; i < num_problems && B->fused; ++i) {
     B->fused = B->loops[i]->fuses_run();
-    // ... and no other problem has this one's iterate
+    // ... and no other problem has this one's iterate or output
+    const uint64_t n = uint64_t(descs[i].num_points[0]) * descs[i].point_dim[0];
     for (uint32_t j = 0; j < num_problems && B->fused; ++j)
-      B->fused = i == j || B->loops[j]->keeps_off(descs[i].point_data[0],
-                                                  uint64_t(descs[i].num_points[0]) *
-                                                      descs[i].point_dim[0]);
+      B->fused = i == j || (B->loops[j]->keeps_off(descs[i].point_data[0], n) &&
+                            B->loops[j]->keeps_off(descs[i].point_data_out, n));
   }
   // work items, largest problems first (longest jobs first balances the tail)
   std::vector<uint32_t> order(num_problems);

@@ -3,7 +3,7 @@ over the kernels that have a form of their own for them."""
 import numpy as np
 import pytest
 
-from cuda_fot_amd import DeviceArray, Loop, capi
+from cuda_fot_amd import DeviceArray, Loop, capi, lulesh_problem
 from helpers import airfoil_problem, assert_bitwise, mine_problem
 
 pytestmark = pytest.mark.gpu
@@ -54,3 +54,61 @@ def test_mine_run_forms(gpu, flags, soa):
         got = run_and_steps(p, capi.functor(capi.KERNEL_MINE, 2, 4, 4), flags, iters, True)
         for g in got[:3]:
             assert_bitwise(g, got[3], f"flags {flags} iters {iters}")
+
+
+class Place:
+    """Part of another buffer, as a loop takes an array."""
+
+    def __init__(self, buffer, first, shape):
+        self.buffer, self.ptr, self.shape = buffer, buffer.ptr + 8 * first, shape
+
+
+@pytest.mark.parametrize("iters", [1, 2])
+def test_run_whose_output_is_another_input(gpu, iters):
+    """The output is the buffer of the node coordinates, which the loop reads:
+    the copy into it comes before the first step."""
+    p = lulesh_problem(5, 4, 6, block_size=32)
+    f = capi.functor(capi.KERNEL_LULESH)
+    got = []
+    for whole in (True, False):
+        force, xyz = (DeviceArray.from_host(d) for d in p.point_data)
+        cells = [DeviceArray.from_host(c) for c in p.cell_data]
+        loop = Loop(f, p.maps, p.num_points, [force, xyz], xyz, cells, block_size=32,
+                    flags=capi.LOOP_TWO_PHASE)
+        if whole:
+            loop.run(iters)
+        else:
+            capi.call("fot_copy", xyz.ptr, force.ptr, xyz.nbytes, None)
+            for _ in range(iters):
+                loop.step()
+            capi.call("fot_copy", force.ptr, xyz.ptr, xyz.nbytes, None)
+        got.append((force.download(), xyz.download()))
+        loop.close()
+    for a, b in zip(*got):
+        assert_bitwise(a, b, f"iters {iters}")
+
+
+@pytest.mark.parametrize("iters", [1, 2])
+@pytest.mark.parametrize("inside", ["output", "iterate", "coordinates"])
+def test_run_whose_cell_output_lies_in_point_data(gpu, inside, iters):
+    """The element volumes are written inside another array: after every step
+    has read and written it."""
+    p = lulesh_problem(5, 4, 6, block_size=32)
+    f, nc = capi.functor(capi.KERNEL_LULESH), p.num_cells
+    got = []
+    for overlap in (True, False):
+        force, xyz = (DeviceArray.from_host(d) for d in p.point_data)
+        out = DeviceArray.from_host(np.zeros_like(p.point_data[0]))
+        sigma = DeviceArray.from_host(p.cell_data[0])
+        into = dict(output=out, iterate=force, coordinates=xyz)[inside]
+        volume = Place(into, 7, (1, nc)) if overlap else DeviceArray.from_host(p.cell_data[1])
+        loop = Loop(f, p.maps, p.num_points, [force, xyz], out, [sigma, volume], block_size=32,
+                    flags=capi.LOOP_TWO_PHASE)
+        loop.run(iters)
+        arrays = dict(iterate=force.download(), output=out.download(), coordinates=xyz.download())
+        if not overlap:
+            arrays[inside].reshape(-1)[7:7 + nc] = volume.download().reshape(-1)
+        got.append(arrays)
+        loop.close()
+    for k in got[0]:
+        assert_bitwise(got[0][k], got[1][k], f"{k}, volumes in {inside}")
