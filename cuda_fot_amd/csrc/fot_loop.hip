@@ -3262,6 +3262,10 @@ bool fot_loop::fuses_run() const {
   if (!(two_phase && gather) &&
       !(owner && !jacobi && (f.kernel != FOT_KERNEL_RES_CALC || owner_gather)))
     return false;
+  // res_calc's owner kernels move AOS rows of four values as two 16-byte halves
+  if (owner && f.kernel == FOT_KERNEL_RES_CALC && !desc.soa &&
+      reinterpret_cast<uintptr_t>(desc.point_data[0]) % 16)
+    return false;
   // and the iterate, the output and the cell output are nobody else's: the
   // copies come before anything is read and the cell output after everything
   // is written, which no longer holds once they are part of a step

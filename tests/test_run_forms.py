@@ -112,3 +112,28 @@ def test_run_whose_cell_output_lies_in_point_data(gpu, inside, iters):
         loop.close()
     for k in got[0]:
         assert_bitwise(got[0][k], got[1][k], f"{k}, volumes in {inside}")
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+def test_owner_res_calc_run_on_an_iterate_of_any_alignment(gpu, aligned):
+    """An iterate that starts on an odd multiple of 8 bytes: the copies take it,
+    the step's 16-byte loads and stores do not touch it."""
+    p = airfoil_problem(nx=20, ny=13, res0_seed=5)
+    n = p.point_data[0].size
+    dev = [DeviceArray.from_host(d) for d in p.point_data]
+    room = DeviceArray.from_host(np.concatenate([[7.0], p.point_data[0].reshape(-1), [9.0]]))
+    if not aligned:
+        dev[0] = Place(room, 1, p.point_data[0].shape)
+        assert dev[0].ptr % 16 == 8
+    out = DeviceArray.from_host(np.full_like(p.point_data[0], np.nan))
+    loop = Loop(capi.functor(capi.KERNEL_RES_CALC), p.maps, p.num_points, dev, out, (),
+                block_size=128, flags=GATHER | capi.LOOP_TWO_PER_THREAD)
+    loop.run(2)
+    got = dev[0].download() if aligned else room.download()[1:n + 1].reshape(-1, 4)
+    ref = run_and_steps(p, capi.functor(capi.KERNEL_RES_CALC), GATHER | capi.LOOP_TWO_PER_THREAD,
+                        2, False)[3]
+    assert_bitwise(got, ref, "iterate")
+    assert_bitwise(out.download(), ref, "output")
+    if not aligned:
+        assert room.download()[0] == 7.0 and room.download()[n + 1] == 9.0
+    loop.close()
