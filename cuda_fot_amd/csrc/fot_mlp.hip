@@ -209,8 +209,9 @@ __device__ __forceinline__ float step_colsum(const float *v) {
 // Forward, loss and backward of the rows of tiles blockIdx.x, + gridDim.x,
 // ...; part[blockIdx.x][params] gets the workgroup's sums of the gradients,
 // loss_part[blockIdx.x] its sum of mask (y - t)^2.  Four waves; wave w owns
-// columns 16 w .. 16 w + 15 of each layer.  Rows past the end carry zeros:
-// their gradients are set to zero whatever the weights are.  IN: the inputs
+// columns 16 w .. 16 w + 15 of each layer.  Rows past the end carry zeros
+// through every layer, whatever the biases are: their products with the zero
+// gradients must not be 0 x infinity.  IN: the inputs
 // rounded up to 32 or 64 (half the first layer's products at 24 inputs).
 template <uint32_t IN>
 __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *__restrict__ p,
@@ -248,14 +249,14 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *
 #pragma unroll
     for (uint32_t v = 0; v < 4; ++v) {
       const float z = a[v] + b1;
-      h1[(4 * q + v) * S + col] = z > 0.f ? z : 0.f;
+      h1[(4 * q + v) * S + col] = z > 0.f && 4 * q + v < n ? z : 0.f;
     }
     __syncthreads();
     a = step_mfma<W>(zero, h1, S, 1, w2 + 16 * w * S, 1, S, lane);
 #pragma unroll
     for (uint32_t v = 0; v < 4; ++v) {
       const float z = a[v] + b2;
-      h2[(4 * q + v) * S + col] = z > 0.f ? z : 0.f;
+      h2[(4 * q + v) * S + col] = z > 0.f && 4 * q + v < n ? z : 0.f;
     }
     __syncthreads();
     // the one output tile: each wave a quarter of its sum, through d1

@@ -134,3 +134,29 @@ def test_mlp_step_at_tile_edges(gpu, n_in, hidden, n_out, rows, masked):
     assert np.all(np.abs(step) <= 3.1e-3)
     sure = np.abs(gr + 0.1 * p) > 0.2 * np.abs(gr + 0.1 * p).max()
     assert np.all(step[sure] * (gr + 0.1 * p)[sure] < 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [15, 16, 17, 31])
+def test_mlp_step_rows_past_the_end_stay_out(gpu, rows):
+    """Weights with which an input of zeros overflows the second layer and the
+    given rows do not: the rows that fill up the last tile add nothing."""
+    from cuda_fot_amd.mlp import MLP
+    n_in, hidden, n_out = 3, 20, 5
+    net = MLP(n_in, hidden, n_out, seed=1)
+    p = net.get_params()
+    w1, b1 = hidden * n_in, hidden
+    p[:w1] = -1e30 / n_in       # with x = 1: exactly cancelled by the bias or below
+    p[w1:w1 + b1] = 0.9e30
+    p[w1 + b1:w1 + b1 + hidden * hidden] = 1e12
+    p[w1 + b1 + hidden * hidden:w1 + b1 + hidden * hidden + hidden] = 0.5
+    net.set_params(p)
+    x = np.ones((rows, n_in), np.float32)
+    t = np.random.default_rng(rows).normal(size=(rows, n_out)).astype(np.float32)
+    loss, g = net.loss_grad(x, t, None)
+    lr, gr = MO.loss_grad(p.astype(np.float64), x, t, None, n_in, hidden, n_out)
+    assert np.isfinite(g).all() and abs(loss - lr) <= 1e-5 * lr
+    # FP32 sums of up to 31 rows and 20 units: 64 roundings of the terms'
+    # magnitudes, which weights and hidden values below 1 scale down
+    y, _ = MO.forward(p.astype(np.float64), x, n_in, hidden, n_out)
+    np.testing.assert_allclose(g, gr, atol=64 * 2.0 ** -24 * 2 * np.abs(y - t).mean(), rtol=0)
