@@ -220,11 +220,12 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *
                                                        const float *__restrict__ mask,
                                                        uint32_t rows, float inv_count,
                                                        float *__restrict__ part,
-                                                       float *__restrict__ loss_part) {
+                                                       double *__restrict__ loss_part) {
   constexpr uint32_t S = kStepStride, W = kStepWidth;
   __shared__ float w1[W * S], w2[W * S], w3[kStepOutputs * S];
   __shared__ float xs[kStepRows * S], h1[kStepRows * S], h2[kStepRows * S];
   __shared__ float d1[kStepRows * S], d2[kStepRows * S], dy[kStepRows * 20];
+  __shared__ double wave_loss[4];
   const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6, r = lane & 15u, q = lane >> 4;
   const uint32_t col = 16 * w + r; // this lane's column of a hidden layer
   step_load<W>(w1, p, s.H, s.I, t);
@@ -237,7 +238,8 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *
   v4f g1[IN / 16], g2[4] = {zero, zero, zero, zero}, g3 = zero;
 #pragma unroll
   for (uint32_t j = 0; j < IN / 16; ++j) g1[j] = zero;
-  float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, loss = 0.f;
+  float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f;
+  double loss = 0.0; // as many FP32 terms per thread as tiles: summed in FP64
   for (uint32_t row0 = blockIdx.x * kStepRows; row0 < rows; row0 += gridDim.x * kStepRows) {
     const uint32_t n = min(kStepRows, rows - row0);
     step_load<kStepRows>(xs, X + size_t(row0) * s.I, n, s.I, t);
@@ -316,9 +318,10 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *
   if (w == 0 && q == 0 && r < s.O) g[s.b3() + r] = gb3;
 #pragma unroll
   for (uint32_t o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
-  if (lane == 0) xs[w] = loss;
+  if (lane == 0) wave_loss[w] = loss;
   __syncthreads();
-  if (t == 0) loss_part[blockIdx.x] = (xs[0] + xs[1]) + (xs[2] + xs[3]);
+  if (t == 0)
+    loss_part[blockIdx.x] = (wave_loss[0] + wave_loss[1]) + (wave_loss[2] + wave_loss[3]);
 }
 
 // Sums the workgroups' gradient parts (in FP64, four slices of them per
@@ -326,7 +329,7 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(MlpShape s, const float *
 // workgroup also sums the loss.  64 parameters per workgroup.
 __global__ __launch_bounds__(256) void mlp_update_kernel(
     float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-    const float *__restrict__ part, const float *__restrict__ loss_part, uint32_t n,
+    const float *__restrict__ part, const double *__restrict__ loss_part, uint32_t n,
     uint32_t parts, float lr_t, float b1, float b2, float eps, float wd, float count,
     float *__restrict__ grad, float *__restrict__ loss) {
   __shared__ double sum[256];
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(256) void mlp_update_kernel(
   }
   if (!loss || blockIdx.x + 1 != gridDim.x) return;
   __syncthreads();
-  sum[t] = t < parts ? double(loss_part[t]) : 0.0; // parts <= kStepBlocks
+  sum[t] = t < parts ? loss_part[t] : 0.0; // parts <= kStepBlocks
   __syncthreads();
   for (uint32_t o = 128; o > 0; o >>= 1) {
     if (t < o) sum[t] += sum[t + o];
@@ -402,7 +405,8 @@ struct fot_mlp {
   float *dY = nullptr, *dH2 = nullptr, *dH1 = nullptr, *part = nullptr;
   // two-launch training steps: gradient and loss parts of the workgroups, the
   // epochs' losses
-  float *gpart = nullptr, *lpart = nullptr, *losses = nullptr;
+  float *gpart = nullptr, *losses = nullptr;
+  double *lpart = nullptr;
   uint32_t gcap = 0, lcap = 0;
   uint64_t step = 0;
   std::vector<void *> owned;
@@ -410,11 +414,11 @@ struct fot_mlp {
   ~fot_mlp() {
     for (void *q : owned) (void)hipFree(q);
   }
-  fot_status alloc(float **q, size_t n) {
+  template <class T> fot_status alloc(T **q, size_t n) {
     void *r = nullptr;
-    FOT_HIP(hipMalloc(&r, std::max<size_t>(1, n) * sizeof(float)));
+    FOT_HIP(hipMalloc(&r, std::max<size_t>(1, n) * sizeof(T)));
     owned.push_back(r);
-    *q = static_cast<float *>(r);
+    *q = static_cast<T *>(r);
     return FOT_OK;
   }
   fot_status reserve(uint32_t rows) {

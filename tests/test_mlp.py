@@ -160,3 +160,17 @@ def test_mlp_step_rows_past_the_end_stay_out(gpu, rows):
     # magnitudes, which weights and hidden values below 1 scale down
     y, _ = MO.forward(p.astype(np.float64), x, n_in, hidden, n_out)
     np.testing.assert_allclose(g, gr, atol=64 * 2.0 ** -24 * 2 * np.abs(y - t).mean(), rtol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [256, 4096 * 3, 4096 * 11, 4096 * 37 + 256])
+def test_mlp_loss_of_equal_terms_is_the_term(gpu, rows):
+    """Every output misses its target by the same value: the mean of equal FP32
+    terms is the term, to the last bit, however many are summed."""
+    from cuda_fot_amd.mlp import MLP
+    net = MLP(1, 1, 1)
+    net.set_params(np.zeros(net.num_params, np.float32))
+    for value in np.float32([0.1, 1.7, 3.3333]):
+        loss, _ = net.loss_grad(np.ones((rows, 1), np.float32), np.full((rows, 1), value),
+                                None)
+        assert np.float32(loss) == value * value
