@@ -86,26 +86,33 @@ struct RunIO {
   double *cells; // the caller's array for the functor's cell output, or null
                  // (then the plan-order copy)
 };
-// A plain step's argument in its place: the owner kernels of a step neither
-// load nor test what only a run needs.  With one kernel for both, a step of a
-// few blocks paid for it (64x32 airfoil, owner compute: 4.11 us without, 4.38
-// with, 4.17-4.26 as two kernels; a full chip's step is the same).
+// A plain step's argument in its place: a step's kernels neither load nor test
+// what only a run needs.  With one kernel for both, steps paid for it: 64x32
+// airfoil, owner compute, 4.11 us without, 4.38 with, 4.08-4.26 as two kernels;
+// 701x463 airfoil, two-phase with staged inputs, blocks of 256, 19.1, 20.4 and
+// 18.4.
 struct StepIO {};
-FOT_DEV RunIO run_io(const EngineArgs &a, StepIO) { return {a.out, a.out, nullptr, nullptr}; }
-FOT_DEV RunIO run_io(const EngineArgs &, const RunIO &run) { return run; }
+FOT_DEV RunIO run_io(double *out, StepIO) { return {out, out, nullptr, nullptr}; }
+FOT_DEV RunIO run_io(double *, const RunIO &run) { return run; }
 
 // Two-phase writeback of a block's cache entry i (point g, values v): added
 // in place when this block alone touches g, else stored in its partial slot
 // for the merge launch.
 template <uint32_t TD, bool SOA>
-FOT_DEV void writeback_two_phase(const HierDev &h, double *out, uint32_t np, uint32_t entry,
+FOT_DEV void writeback_two_phase(const HierDev &h, const RunIO &io, uint32_t np, uint32_t entry,
                                  uint32_t g, const double *v) {
   const uint32_t s = h.wslot[entry];
   if (s == kExclusive) {
+    double sum[TD];
 #pragma unroll
     for (uint32_t d = 0; d < TD; ++d) {
-      double *p = out + pidx<SOA>(np, g, TD, d);
-      *p = *p + v[d];
+      const size_t at = pidx<SOA>(np, g, TD, d);
+      sum[d] = io.base[at] + v[d];
+      io.out[at] = sum[d];
+    }
+    if (io.also) {
+#pragma unroll
+      for (uint32_t d = 0; d < TD; ++d) io.also[pidx<SOA>(np, g, TD, d)] = sum[d];
     }
   } else {
 #pragma unroll
@@ -119,11 +126,12 @@ FOT_DEV void writeback_two_phase(const HierDev &h, double *out, uint32_t np, uin
 // handed out block by block, so a block's partial stores are contiguous;
 // handing them out point by point instead, contiguous for this launch's
 // reads, measured 5 % slower on hex and mini_aero meshes.)
-template <uint32_t TD, bool SOA>
+template <uint32_t TD, bool SOA, class IO>
 __global__ __launch_bounds__(256) void merge_partials_kernel(
-    RunIO io, uint32_t np, const uint32_t *__restrict__ pt,
+    double *out, IO run, uint32_t np, const uint32_t *__restrict__ pt,
     const uint32_t *__restrict__ off, const uint32_t *__restrict__ slots,
     const double *__restrict__ partial, uint32_t n) {
+  const RunIO io = run_io(out, run);
   const uint32_t j = blockIdx.x * 256u + threadIdx.x;
   if (j >= n) return;
   const uint32_t g = pt[j], s0 = off[j], s1 = off[j + 1];
@@ -345,8 +353,8 @@ constexpr uint32_t kSpinLimit = 1u << 21;
 // each XCD gets a contiguous run of blocks; the single launch hands out
 // tickets in plan (colour-major) order, so every block a workgroup may wait
 // on has already been taken by a running workgroup.
-template <bool DEP>
-FOT_DEV uint32_t pick_block(const DepDev &dd, uint32_t blk_begin, uint32_t nbc, uint32_t &gen) {
+template <bool DEP, class C>
+FOT_DEV uint32_t pick_block(const C &dd, uint32_t blk_begin, uint32_t nbc, uint32_t &gen) {
   if constexpr (!DEP) {
     gen = 0;
     return blk_begin + xcd_block(blockIdx.x, nbc);
@@ -364,8 +372,8 @@ FOT_DEV uint32_t pick_block(const DepDev &dd, uint32_t blk_begin, uint32_t nbc, 
 }
 
 // Waits (first wave) for the lower-colour neighbours of block b.
-template <bool DEP>
-FOT_DEV void wait_predecessors(const DepDev &dd, uint32_t b, uint32_t gen) {
+template <bool DEP, class C>
+FOT_DEV void wait_predecessors(const C &dd, uint32_t b, uint32_t gen) {
   if constexpr (DEP) {
     if (threadIdx.x < 64) {
       const uint32_t d0 = dd.dep_off[b], nd = dd.dep_off[b + 1] - d0;
@@ -389,8 +397,8 @@ FOT_DEV void wait_predecessors(const DepDev &dd, uint32_t b, uint32_t gen) {
 
 // Publishes block b's writeback; the last block of the launch re-arms the
 // ticket counter for the next launch.
-template <bool DEP>
-FOT_DEV void publish(const DepDev &dd, uint32_t b, uint32_t gen) {
+template <bool DEP, class C>
+FOT_DEV void publish(const C &dd, uint32_t b, uint32_t gen) {
   if constexpr (DEP) {
     __builtin_amdgcn_s_waitcnt(0); // this wave's stores are in L2
     __syncthreads();
@@ -413,15 +421,17 @@ FOT_DEV void publish(const DepDev &dd, uint32_t b, uint32_t gen) {
 // loaded once per block point into LDS after the cache, and the functor reads
 // it there by block-local id instead of gathering it per cell.  NTC: the
 // functor's read-once cell data loaded with nontemporal hints
-// (StreamCellArgs; the same values).
-template <class F, bool SOA, int MODE, int LB = 1024, bool STG = false, bool NTC = false>
+// (StreamCellArgs; the same values).  CTL: a DepDev, or in mode 2 a StepIO or
+// RunIO.
+template <class F, bool SOA, int MODE, class CTL, int LB = 1024, bool STG = false,
+          bool NTC = false>
 __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_hier_kernel(
-    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, DepDev dd,
+    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, CTL ctl,
     uint32_t blk_begin, uint32_t nbc) {
   constexpr bool DEP = MODE == 1;
   extern __shared__ double cache[];
   uint32_t gen;
-  const uint32_t b = pick_block<DEP>(dd, blk_begin, nbc, gen);
+  const uint32_t b = pick_block<DEP>(ctl, blk_begin, nbc, gen);
   const uint32_t tid = threadIdx.x;
   const uint32_t e0 = h.blk_cell_off[b], ne = h.blk_cell_off[b + 1] - e0;
   const uint32_t c0 = h.blk_cache_off[b], m = h.blk_cache_off[b + 1] - c0;
@@ -468,7 +478,7 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_h
     if (colour == c) add_to_cache<F>(cache, m, loc, inc);
     __syncthreads();
   }
-  wait_predecessors<DEP>(dd, b, gen);
+  wait_predecessors<DEP>(ctl, b, gen);
   // (loading the first two write-back entries per thread, their ids, slots
   // and in-place output values, before the accumulation measured slower on
   // hex 128^3: 150 -> 179 us at B = 512, two-phase)
@@ -479,7 +489,7 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_h
       double v[F::TD];
 #pragma unroll
       for (uint32_t d = 0; d < F::TD; ++d) v[d] = cache[d * m + i];
-      writeback_two_phase<F::TD, SOA>(h, a.out, np, c0 + i, g, v);
+      writeback_two_phase<F::TD, SOA>(h, run_io(a.out, ctl), np, c0 + i, g, v);
     } else {
 #pragma unroll
       for (uint32_t d = 0; d < F::TD; ++d) {
@@ -488,7 +498,7 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_h
       }
     }
   }
-  publish<DEP>(dd, b, gen);
+  publish<DEP>(ctl, b, gen);
 }
 
 // ---- gather accumulation ----------------------------------------------------
@@ -571,10 +581,11 @@ template <class F, bool SOA> struct RowIds {
 // R: rounds of points a thread takes (at most R * blockDim.x cached points).
 // Without write slots (one launch per block colour) every point is added in
 // place.
-template <class F, bool SOA, int R, int LB = 1024, bool NTC = false>
+template <class F, bool SOA, int R, class IO, int LB = 1024, bool NTC = false>
 __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_gather_kernel(
-    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, RunIO io,
+    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, IO run,
     uint32_t blk_begin, uint32_t nbc) {
+  const RunIO io = run_io(a.out, run);
   constexpr uint32_t MD = F::MD, TD = F::TD, PD = std::min(kPassDims<F>, TD);
   extern __shared__ double lds[];
   const uint4 rec = h.rec[blk_begin + xcd_block(blockIdx.x, nbc)];
@@ -703,15 +714,15 @@ __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_g
 // res_calc hierarchical with the block's cells' q and adt staged in LDS next
 // to the res cache (they are read through the same mapping-0 points), so
 // the edge loop gathers only x from HBM.
-template <bool SOA, int MODE>
+template <bool SOA, int MODE, class CTL>
 __global__ __launch_bounds__(1024) void res_calc_hier_staged_kernel(EngineArgs a, HierDev h,
-                                                                    DepDev dd,
+                                                                    CTL ctl,
                                                                     uint32_t blk_begin,
                                                                     uint32_t nbc) {
   constexpr bool DEP = MODE == 1;
   extern __shared__ double lds[];
   uint32_t gen;
-  const uint32_t b = pick_block<DEP>(dd, blk_begin, nbc, gen);
+  const uint32_t b = pick_block<DEP>(ctl, blk_begin, nbc, gen);
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
   const uint32_t e0 = h.blk_cell_off[b], ne = h.blk_cell_off[b + 1] - e0;
   const uint32_t c0 = h.blk_cache_off[b], m = h.blk_cache_off[b + 1] - c0;
@@ -780,14 +791,14 @@ __global__ __launch_bounds__(1024) void res_calc_hier_staged_kernel(EngineArgs a
     }
     __syncthreads();
   }
-  wait_predecessors<DEP>(dd, b, gen);
+  wait_predecessors<DEP>(ctl, b, gen);
   if constexpr (MODE == 2) {
     for (uint32_t i = tid; i < m; i += bd) {
       const uint32_t g = i == tid ? g0 : h.cached[c0 + i];
       double v[4];
 #pragma unroll
       for (uint32_t d = 0; d < 4; ++d) v[d] = res_s[d * m + i];
-      writeback_two_phase<4, SOA>(h, a.out, np, c0 + i, g, v);
+      writeback_two_phase<4, SOA>(h, run_io(a.out, ctl), np, c0 + i, g, v);
     }
     return;
   }
@@ -813,17 +824,18 @@ __global__ __launch_bounds__(1024) void res_calc_hier_staged_kernel(EngineArgs a
       o[1] = make_double2(r[2], r[3]);
     }
   }
-  publish<DEP>(dd, b, gen);
+  publish<DEP>(ctl, b, gen);
 }
 
 // The same with gathered sums (see eng_gather_kernel), for launches per block
 // colour and two-phase ones: an edge stores its flux f, and a point's list names
 // the fluxes it adds or, as the edge's second cell, subtracts (place | 0x8000;
 // its increment is -f, and v + (-f) is v - f).
-template <bool SOA, int R>
+template <bool SOA, int R, class IO>
 __global__ __launch_bounds__(1024) void res_calc_hier_gather_kernel(EngineArgs a, HierDev h,
-                                                                    RunIO io, uint32_t blk_begin,
+                                                                    IO run, uint32_t blk_begin,
                                                                     uint32_t nbc) {
+  const RunIO io = run_io(a.out, run);
   extern __shared__ double lds[];
   const uint4 rec = h.rec[blk_begin + xcd_block(blockIdx.x, nbc)];
   const uint32_t tid = threadIdx.x, T = blockDim.x, e0 = rec.x, ne = rec.y, c0 = rec.z, m = rec.w;
@@ -1128,14 +1140,14 @@ template <class F, bool SOA, class IO>
 __global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, HierDev h,
                                                                uint32_t nb, IO run) {
   extern __shared__ double lds[];
-  owner_gather_block<F, SOA>(a, h, run_io(a, run), h.items[xcd_block(blockIdx.x, nb)], lds);
+  owner_gather_block<F, SOA>(a, h, run_io(a.out, run), h.items[xcd_block(blockIdx.x, nb)], lds);
 }
 
 template <class F, bool SOA, class IO, int LB = 1024>
 __global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, uint32_t nb,
                                                        IO run) {
   extern __shared__ double lds[];
-  owner_block<F, SOA>(a, h, run_io(a, run), xcd_block(blockIdx.x, nb), lds);
+  owner_block<F, SOA>(a, h, run_io(a.out, run), xcd_block(blockIdx.x, nb), lds);
 }
 
 // One problem of a batch: its engine arguments and owner-compute plan.
@@ -1699,7 +1711,7 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_kernel(EngineArgs a,
                                                                const uint32_t *__restrict__ plist,
                                                                uint32_t nb, IO run) {
   extern __shared__ double lds[];
-  const RunIO io = run_io(a, run);
+  const RunIO io = run_io(a.out, run);
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
@@ -1718,7 +1730,7 @@ __global__ __launch_bounds__(1024) void res_calc_owner3_stream_kernel(
     const uint32_t *__restrict__ packed, const uint32_t *__restrict__ plist, uint32_t nb,
     IO run) {
   extern __shared__ double lds[];
-  const RunIO io = run_io(a, run);
+  const RunIO io = run_io(a.out, run);
   const uint32_t b = xcd_block(blockIdx.x, nb);
   const OwnerMeta mt = meta[b];
   const uint32_t tid = threadIdx.x, bd = blockDim.x;
@@ -1743,7 +1755,7 @@ __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
                                                                const uint32_t *__restrict__ plist,
                                                                uint32_t nb, IO run) {
   extern __shared__ double lds[];
-  const RunIO io = run_io(a, run);
+  const RunIO io = run_io(a.out, run);
   const uint32_t tid = threadIdx.x, bd = blockDim.x, G = gridDim.x;
   uint32_t j = blockIdx.x;
   if (j >= nb) return;
@@ -1855,9 +1867,9 @@ bool reads_iterate(const fot_functor &f) { return f.kernel == FOT_KERNEL_MINE; }
 // Launches eng_hier_kernel<F, SOA, MODE>: the small-bound instantiation when
 // the blocks fit it, the staged-input one when asked and the functor has a
 // staged input.
-template <class F, bool SOA, int MODE>
+template <class F, bool SOA, int MODE, class CTL>
 void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
-                     const EngineArgs &a, const HierDev &h, const DepDev &dd, uint32_t b0,
+                     const EngineArgs &a, const HierDev &h, const CTL &ctl, uint32_t b0,
                      uint32_t nbc, bool stream_cells = false) {
   constexpr bool CAN = StagedInput<F>::slot >= 0;
   constexpr int SB = kSmallBound<F>;
@@ -1865,11 +1877,11 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
     if (stream_cells && !stage) {
       const StreamCellArgs sa{a};
       if (threads <= uint32_t(SB))
-        hipLaunchKernelGGL((eng_hier_kernel<F, SOA, 2, SB, false, true>), dim3(grid),
-                           dim3(threads), lds, s, sa, h, dd, b0, nbc);
+        hipLaunchKernelGGL((eng_hier_kernel<F, SOA, 2, CTL, SB, false, true>), dim3(grid),
+                           dim3(threads), lds, s, sa, h, ctl, b0, nbc);
       else
-        hipLaunchKernelGGL((eng_hier_kernel<F, SOA, 2, 1024, false, true>), dim3(grid),
-                           dim3(threads), lds, s, sa, h, dd, b0, nbc);
+        hipLaunchKernelGGL((eng_hier_kernel<F, SOA, 2, CTL, 1024, false, true>), dim3(grid),
+                           dim3(threads), lds, s, sa, h, ctl, b0, nbc);
       return;
     }
   }
@@ -1877,25 +1889,25 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
     if (threads <= uint32_t(SB)) {
       if constexpr (CAN) {
         if (stage) {
-          hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, SB, true>), dim3(grid),
-                             dim3(threads), lds, s, a, h, dd, b0, nbc);
+          hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, CTL, SB, true>), dim3(grid),
+                             dim3(threads), lds, s, a, h, ctl, b0, nbc);
           return;
         }
       }
-      hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, SB, false>), dim3(grid), dim3(threads),
-                         lds, s, a, h, dd, b0, nbc);
+      hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, CTL, SB, false>), dim3(grid), dim3(threads),
+                         lds, s, a, h, ctl, b0, nbc);
       return;
     }
   }
   if constexpr (CAN) {
     if (stage) {
-      hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, 1024, true>), dim3(grid), dim3(threads),
-                         lds, s, a, h, dd, b0, nbc);
+      hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, CTL, 1024, true>), dim3(grid), dim3(threads),
+                         lds, s, a, h, ctl, b0, nbc);
       return;
     }
   }
-  hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, 1024, false>), dim3(grid), dim3(threads),
-                     lds, s, a, h, dd, b0, nbc);
+  hipLaunchKernelGGL((eng_hier_kernel<F, SOA, MODE, CTL, 1024, false>), dim3(grid), dim3(threads),
+                     lds, s, a, h, ctl, b0, nbc);
 }
 
 // Launches eng_owner_gather_kernel or eng_owner_kernel; IO: StepIO or RunIO.
@@ -1919,9 +1931,9 @@ void launch_owner(bool gather, uint32_t nb, uint32_t threads, uint32_t lds, hipS
 }
 
 // Launches eng_gather_kernel<F, SOA, R>.
-template <class F, bool SOA, int R>
+template <class F, bool SOA, int R, class IO>
 void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
-                   const EngineArgs &a, const HierDev &h, const RunIO &io, uint32_t b0,
+                   const EngineArgs &a, const HierDev &h, const IO &io, uint32_t b0,
                    uint32_t nbc, bool stream_cells) {
   constexpr int SB = kSmallBound<F>;
   const bool small = threads <= uint32_t(SB);
@@ -1929,19 +1941,19 @@ void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
     if (stream_cells) {
       const StreamCellArgs sa{a};
       if (small)
-        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB, true>), dim3(grid), dim3(threads),
+        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, IO, SB, true>), dim3(grid), dim3(threads),
                            lds, s, sa, h, io, b0, nbc);
       else
-        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, 1024, true>), dim3(grid), dim3(threads),
+        hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, IO, 1024, true>), dim3(grid), dim3(threads),
                            lds, s, sa, h, io, b0, nbc);
       return;
     }
   }
   if (small)
-    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, SB>), dim3(grid), dim3(threads), lds, s, a, h,
+    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, IO, SB>), dim3(grid), dim3(threads), lds, s, a, h,
                        io, b0, nbc);
   else
-    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R>), dim3(grid), dim3(threads), lds, s, a, h,
+    hipLaunchKernelGGL((eng_gather_kernel<F, SOA, R, IO>), dim3(grid), dim3(threads), lds, s, a, h,
                        io, b0, nbc);
 }
 
@@ -2128,6 +2140,11 @@ struct fot_loop {
   fot_status build_atomic();
   fot_status build_global_colour();
   fot_status build_hierarchical();
+  // launches nb plan blocks from b0 on: their gather kernel, or what `colours`
+  // launches
+  template <class F, bool SOA, class IO, class Colours>
+  void launch_blocks(uint32_t nb, hipStream_t s, const IO &io, uint32_t b0, bool stream_cells,
+                     Colours &&colours) const;
   // one step, adding in place, or as `run` says (where fuses_run allows it)
   fot_status enqueue(hipStream_t s, const RunIO *run = nullptr);
   // whether fot_loop_run's copies can be part of its first and last step
@@ -2277,6 +2294,21 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
   });
   if (st != FOT_OK) return st;
   if (stage_pd && !stages) return FOT_OK; // eng_hier_kernel stages the others' input
+  // Cells of two points: the colour loop where a block's points add few
+  // increments each.  A gathering point reads its list's empty places too, and
+  // its row goes through LDS whether one cell reads it or four.  Blocks of
+  // consecutive cells on a GPS-ordered mesh have 1.4 to 2.2 increments per
+  // point.  AOS, colour loop / gathered, a two-phase step: volna, 1.27 M edges
+  // in blocks of 512, 48.8 / 57.7 us; airfoil 1100x550 35.6 / 39.3; mini_aero
+  // 55^3, blocks of 128, 41.2 / 47.7 (per colour 86 / 100).  Around 2.4 they are
+  // level (mini_aero 55^3 in blocks of 256 76.3 / 75.1 per colour), from 2.5 on
+  // gathered is faster, by 2 to 20 % on compact parts (2.5 to 3.6).  In SOA it is
+  // faster per colour at any ratio (2 to 30 %), and two-phase but for large plans
+  // of the lowest (volna, 1.27 M edges in blocks of 512: 49.9 / 54.1).
+  if (md == 2 && !staged && !stage_pd) {
+    const double per_point = double(loc.size()) / blk_cache_off[nb];
+    if (desc.soa ? two_phase && nb > 1024 && per_point < 1.6 : per_point < 2.4) return FOT_OK;
+  }
   // res_calc_hier_gather_kernel, where the plan's blocks do not fill the chip
   // for one round and their latency is what counts (colour loop / this, a
   // step: 64x32 8.9 / 7.2 us, 200x150 10.0 / 7.6, blocks of 512; 701x463,
@@ -2962,9 +2994,29 @@ template <class F> uint32_t atomic_threads(uint32_t cells) {
   return n;
 }
 
+template <class F, bool SOA, class IO, class Colours>
+void fot_loop::launch_blocks(uint32_t nb, hipStream_t s, const IO &io, uint32_t b0,
+                             bool stream_cells, Colours &&colours) const {
+  if (!gather) {
+    colours();
+    return;
+  }
+  if constexpr (std::is_same<F, ResCalcF>::value) {
+    if (staged) {
+      hipLaunchKernelGGL((gather_rounds == 1 ? res_calc_hier_gather_kernel<SOA, 1, IO>
+                                             : res_calc_hier_gather_kernel<SOA, 2, IO>),
+                         dim3(nb), dim3(threads), lds_bytes, s, plan_args, hier, io, b0, nb);
+      return;
+    }
+  }
+  if (gather_rounds == 1)
+    launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, io, b0, nb, stream_cells);
+  else
+    launch_gather<F, SOA, 2>(nb, threads, lds_bytes, s, plan_args, hier, io, b0, nb, stream_cells);
+}
+
 fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
   if (desc.num_cells == 0) return FOT_OK; // nothing to launch
-  const RunIO io = run ? *run : RunIO{base.out, base.out, nullptr, nullptr};
   const fot_status st = dispatch(&f, desc.soa, [&]<class F, bool SOA>() -> fot_status {
     const uint32_t bs = cfg.block_size;
     // direct launches: one thread per cell, whatever the block size
@@ -3011,7 +3063,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
           const OwnerMeta *om = owner_meta;
           const uint32_t *pc = hier.cached, *pp = hier.packed, *pl = owner_plist;
           uint32_t nbv = nb;
-          RunIO iov = io; // (a StepIO takes its first byte)
+          RunIO iov = run ? *run : RunIO{}; // (a StepIO takes its first byte)
           void *kargs[] = {&pa, &om, &pc, &pp, &pl, &nbv, &iov};
           FOT_HIP(hipLaunchKernel(run ? owner3_run_fn : owner3_fn, dim3(launch_grid),
                                   dim3(threads), kargs, size_t(lds_bytes), s));
@@ -3026,7 +3078,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
 #undef FOT_OWNER2
 #undef FOT_OWNER2P
       } else {
-        if (run) launch_owner<F, SOA>(gather, nb, threads, lds_bytes, s, plan_args, hier, io);
+        if (run) launch_owner<F, SOA>(gather, nb, threads, lds_bytes, s, plan_args, hier, *run);
         else launch_owner<F, SOA>(gather, nb, threads, lds_bytes, s, plan_args, hier, StepIO{});
       }
     } else if (dep_order) {
@@ -3035,7 +3087,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
       bool done = false;
       if constexpr (std::is_same<F, ResCalcF>::value) {
         if (staged) {
-          hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 1>), dim3(nb), dim3(threads),
+          hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 1, DepDev>), dim3(nb), dim3(threads),
                              lds_bytes, s, plan_args, hier, dep, 0u, nb);
           done = true;
         }
@@ -3046,56 +3098,41 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
     } else if (two_phase) {
       // every block in one launch, then the merge of the shared points
       const uint32_t nb = colour_blk_off.back();
-      bool done = false;
-      if constexpr (std::is_same<F, ResCalcF>::value) {
-        if (staged && gather) {
-          hipLaunchKernelGGL((gather_rounds == 1 ? res_calc_hier_gather_kernel<SOA, 1>
-                                                 : res_calc_hier_gather_kernel<SOA, 2>),
-                             dim3(nb), dim3(threads), lds_bytes, s, plan_args, hier, io, 0u, nb);
-          done = true;
-        } else if (staged) {
-          hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 2>), dim3(nb), dim3(threads),
-                             lds_bytes, s, plan_args, hier, dep, 0u, nb);
-          done = true;
-        }
-      }
-      if (gather && !done) {
-        if (gather_rounds == 1)
-          launch_gather<F, SOA, 1>(nb, threads, lds_bytes, s, plan_args, hier, io, 0u, nb, nontemporal);
-        else
-          launch_gather<F, SOA, 2>(nb, threads, lds_bytes, s, plan_args, hier, io, 0u, nb, nontemporal);
-      } else if (!done)
-        launch_eng_hier<F, SOA, 2>(stage_pd, nb, threads, lds_bytes, s, plan_args, hier, dep,
-                                   0u, nb, nontemporal);
-      if (merge_n)
-        hipLaunchKernelGGL((merge_partials_kernel<F::TD, SOA>), dim3((merge_n + 255) / 256),
-                           dim3(256), 0, s, io, plan_args.num_points[0], merge_pt,
-                           merge_off, merge_slots, hier.partial, merge_n);
+      auto launch = [&](const auto &io) {
+        using IO = std::decay_t<decltype(io)>;
+        launch_blocks<F, SOA>(nb, s, io, 0u, nontemporal, [&] {
+          if constexpr (std::is_same<F, ResCalcF>::value) {
+            if (staged) {
+              hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 2, IO>), dim3(nb),
+                                 dim3(threads), lds_bytes, s, plan_args, hier, io, 0u, nb);
+              return;
+            }
+          }
+          launch_eng_hier<F, SOA, 2>(stage_pd, nb, threads, lds_bytes, s, plan_args, hier, io, 0u,
+                                     nb, nontemporal);
+        });
+        if (merge_n)
+          hipLaunchKernelGGL((merge_partials_kernel<F::TD, SOA, IO>), dim3((merge_n + 255) / 256),
+                             dim3(256), 0, s, plan_args.out, io, plan_args.num_points[0],
+                             merge_pt, merge_off, merge_slots, hier.partial, merge_n);
+      };
+      if (run) launch(*run);
+      else launch(StepIO{});
     } else {
       for (size_t c = 0; c + 1 < colour_blk_off.size(); ++c) {
         const uint32_t b0 = colour_blk_off[c], nbc = colour_blk_off[c + 1] - b0;
         if (nbc == 0) continue;
-        if constexpr (std::is_same<F, ResCalcF>::value) {
-          if (staged && gather) {
-            hipLaunchKernelGGL((gather_rounds == 1 ? res_calc_hier_gather_kernel<SOA, 1>
-                                                 : res_calc_hier_gather_kernel<SOA, 2>),
-                               dim3(nbc), dim3(threads), lds_bytes, s, plan_args, hier, io, b0,
-                               nbc);
-            continue;
+        launch_blocks<F, SOA>(nbc, s, StepIO{}, b0, false, [&] {
+          if constexpr (std::is_same<F, ResCalcF>::value) {
+            if (staged) {
+              hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 0, DepDev>), dim3(nbc),
+                                 dim3(threads), lds_bytes, s, plan_args, hier, dep, b0, nbc);
+              return;
+            }
           }
-          if (staged) {
-            hipLaunchKernelGGL((res_calc_hier_staged_kernel<SOA, 0>), dim3(nbc),
-                               dim3(threads), lds_bytes, s, plan_args, hier, dep, b0, nbc);
-            continue;
-          }
-        }
-        if (gather && gather_rounds == 1)
-          launch_gather<F, SOA, 1>(nbc, threads, lds_bytes, s, plan_args, hier, io, b0, nbc, false);
-        else if (gather)
-          launch_gather<F, SOA, 2>(nbc, threads, lds_bytes, s, plan_args, hier, io, b0, nbc, false);
-        else
           launch_eng_hier<F, SOA, 0>(stage_pd, nbc, threads, lds_bytes, s, plan_args, hier, dep,
-                                   b0, nbc);
+                                     b0, nbc);
+        });
       }
     }
     const hipError_t e = hipGetLastError();
@@ -3259,7 +3296,7 @@ bool fot_loop::fuses_run() const {
   // that takes a RunIO; a captured graph's steps add in place
   if (exec || desc.num_cells == 0 || !every_point) return false;
   const bool jacobi = reads_iterate(f);
-  if (!(two_phase && gather) &&
+  if (!two_phase &&
       !(owner && !jacobi && (f.kernel != FOT_KERNEL_RES_CALC || owner_gather)))
     return false;
   // res_calc's owner kernels move AOS rows of four values as two 16-byte halves

@@ -1,0 +1,101 @@
+"""Which hierarchical plans gather their sums, and that either kernel gives the
+oracle's bits.  The rule is restated here on the host plan; the loop's LDS size
+tells which kernel was planned."""
+import numpy as np
+import pytest
+
+import oracle as O
+from cuda_fot_amd import Problem, capi, meshgen, mini_aero_problem, plan, volna_problem
+from helpers import airfoil_problem, assert_bitwise, mine_problem, oracle_of
+
+TP = capi.LOOP_TWO_PHASE
+STAGED_DIM = {O.MINI_AERO: 28, O.LULESH: 3}
+
+
+def host_plan(p, block_size):
+    """Per-block increments per cached point (the mean of the plan), the longest
+    list, the most cached points and the workgroup's threads."""
+    md, cached, most, longest, cells, blocks = p.maps[0].shape[1], 0, 0, 0, 0, 0
+    for c in plan.hplan(p.maps, p.num_points[0], block_size, p.partition_vector):
+        off, ids = c["block_offsets"], c["cell_list"][0].reshape(md, -1)
+        for b in range(len(off) - 1):
+            n = np.bincount(ids[:, off[b]:off[b + 1]].ravel())
+            cached, most, longest = cached + n.size, max(most, n.size), max(longest, n.max())
+            cells, blocks = max(cells, off[b + 1] - off[b]), blocks + 1
+    threads = max(64, -(-int(cells) // 64) * 64)
+    return dict(per_point=p.maps[0].size / cached, longest=int(longest), most=int(most),
+                threads=threads, blocks=blocks)
+
+
+def gathers(p, kernel, h, two_phase):
+    md, td = p.maps[0].shape[1], p.point_data[0].shape[0 if p.soa else 1]
+    if h["longest"] > 8 or h["most"] > 2 * h["threads"]:
+        return False
+    if md == 2:
+        if p.soa:
+            return not (two_phase and h["blocks"] > 1024 and h["per_point"] < 1.6)
+        return h["per_point"] >= 2.4
+    return True
+
+
+def lds_of(p, kernel, h, gather):
+    md, td = p.maps[0].shape[1], p.point_data[0].shape[0 if p.soa else 1]
+    if not gather:
+        return 8 * td * h["most"]
+    dims = td if md == 2 and td <= 5 else 1 if md >= 8 else 8 // md
+    planes = 8 * min(dims, td) * (md * h["threads"] + 1)
+    staged = STAGED_DIM.get(kernel, 0)
+    return max(planes, 8 * (staged | 1) * h["most"] if staged else 0)
+
+
+def check(p, kernel, functor, block_size, iters, expect, flags=(0, TP)):
+    """Runs the loop per colour and two-phase against the oracle's replay, on
+    the kernel expected (a bool, or one per entry of flags)."""
+    h = host_plan(p, block_size)
+    o = oracle_of(p, kernel)
+    o.loop_hier_replay(O.OraclePlan(p.maps, p.num_points[0], block_size, p.partition_vector), iters)
+    start = [None if d is None else d.copy() for d in p.point_data]
+    for k, f in enumerate(flags):
+        want = expect if isinstance(expect, bool) else expect[k]
+        assert gathers(p, kernel, h, f & TP) == want, h
+        p.point_data = [None if d is None else d.copy() for d in start]
+        stats = p.gpu_loop(functor, capi.STRATEGY_HIERARCHICAL, iters, block_size=block_size, flags=f)
+        assert stats["lds_bytes"] == lds_of(p, kernel, h, want), (f, h, stats)
+        assert_bitwise(p.point_data[0], o.target, f"flags {f} {h}")
+    return h
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("kind,block_size,gather", [("airfoil", 128, False), ("airfoil", 256, True),
+                                                    ("mine", 128, False), ("mine", 256, True),
+                                                    ("volna", 128, False), ("volna", 512, True),
+                                                    ("mini_aero", 128, False),
+                                                    ("mini_aero", 512, True)])
+def test_two_point_cells_gather_where_points_add_enough(gpu, kind, block_size, gather, soa):
+    """GPS-ordered meshes on either side of 2.4 increments per cached point: AOS
+    plans below keep the colour loop, SOA plans gather."""
+    if kind == "airfoil":
+        p, kernel, f = airfoil_problem(160, 80, soa=soa, res0_seed=3), O.RES_CALC, capi.KERNEL_RES_CALC
+    elif kind == "mine":
+        p, kernel, f = mine_problem(160, 80, soa=soa), O.MINE2, None
+    elif kind == "volna":
+        p, kernel, f = volna_problem(meshgen.tri_mesh(80, 80, seed=1), soa=soa), O.VOLNA, capi.KERNEL_VOLNA
+    else:
+        p, kernel, f = mini_aero_problem(meshgen.hex_faces(34, 34, 34), soa=soa), O.MINI_AERO, \
+            capi.KERNEL_MINI_AERO
+    p.reorder("gps")
+    f = capi.functor(capi.KERNEL_MINE, 2, 4, 4) if f is None else capi.functor(f)
+    check(p, kernel, f, block_size, 2 if kind == "mine" else 1, gather or soa)
+
+
+@pytest.mark.gpu
+def test_large_soa_plans_of_few_increments_per_point(gpu):
+    p = volna_problem(meshgen.tri_mesh(220, 220, seed=1), soa=True)
+    p.reorder("gps")
+    h = check(p, O.VOLNA, capi.functor(capi.KERNEL_VOLNA), 128, 1, (True, False))
+    assert h["blocks"] > 1024 and h["per_point"] < 1.6
+    p = volna_problem(meshgen.tri_mesh(120, 120, seed=1), soa=True)
+    p.reorder("gps")
+    h = check(p, O.VOLNA, capi.functor(capi.KERNEL_VOLNA), 128, 1, True)
+    assert h["blocks"] <= 1024

@@ -47,11 +47,20 @@ def test_owner_res_calc_run_forms(gpu, form, two, soa):
 
 
 @pytest.mark.parametrize("soa", [False, True])
-@pytest.mark.parametrize("flags", [OWN, capi.LOOP_TWO_PHASE])
-def test_mine_run_forms(gpu, flags, soa):
-    p = mine_problem(N=30, M=17, soa=soa)
+@pytest.mark.parametrize("flags", [OWN, capi.LOOP_TWO_PHASE,
+                                   capi.LOOP_TWO_PHASE | capi.LOOP_STAGE_INPUTS])
+@pytest.mark.parametrize("order", [None, "gps"])  # AOS two-phase: gathered sums, colour loop
+def test_mine_run_forms(gpu, order, flags, soa):
+    p = mine_problem(N=90, M=57, soa=soa, shuffle=False)
+    if order:
+        p.reorder(order)
+    else:
+        p.partition(method="bisect")
+        p.reorder_to_partition()
+        p.renumber_points()
     for iters in (1, 3):
-        got = run_and_steps(p, capi.functor(capi.KERNEL_MINE, 2, 4, 4), flags, iters, True)
+        got = run_and_steps(p, capi.functor(capi.KERNEL_MINE, 2, 4, 4), flags, iters, True,
+                            None if order else p.partition_vector)
         for g in got[:3]:
             assert_bitwise(g, got[3], f"flags {flags} iters {iters}")
 
