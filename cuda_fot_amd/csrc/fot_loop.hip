@@ -1992,7 +1992,9 @@ struct fot_loop {
   uint32_t lds_bytes = 0, threads = 0;
   bool staged = false;
   uint32_t gather_rounds = 1;
-  bool may_gather = true; // off for the problems of a batch that cannot all gather
+  // whether owner blocks gather: as their rule says, or (a batch's problems)
+  // wherever the kernel takes them, or not at all
+  enum class Gather { kByRule, kAlways, kNever } gather_policy = Gather::kByRule;
   bool gather = false;   // hierarchical: points gather their increments (eng_gather_kernel)
   bool stage_pd = false; // generic hierarchical: the functor's staged input in LDS
   bool dep_order = false;
@@ -2406,6 +2408,25 @@ fot_status fot_loop::build_owner_gather(
                                  (most_owned + kOwnerPoints - 1) / kOwnerPoints);
   const uint32_t t = std::max<uint32_t>(64, (most + 63) / 64 * 64);
   if (st != FOT_OK || !takes || t > 512 || md * cap > 0xfffeu || lds > 80u * 1024u) return st;
+  if (gather_policy == Gather::kByRule) {
+    // A loop of its own gathers where two cells per thread make the workgroup
+    // smaller (parts whose points need the threads anyway, colour loop /
+    // gathered: mine on quads 500^2, k-way parts of 256 points, 12.1 / 17.4 us;
+    // getacc 500^2 18.2 / 19.7) and the blocks' ids are consecutive: then a block
+    // is a round trip shorter (64 cases of all sizes: 0.96 to 1.5 times as fast).
+    // With other ids volna loses 2 to 11 % (97 000 edges, GPS-ordered, parts of
+    // 256: 6.6 / 7.2), getacc, which needs none for its cells, still gains, and
+    // AOS mine loses 2 to 7 % on small meshes but gains from some 2^18 runs on
+    // (489 000 edges, parts of 256, 11.3 / 10.6).
+    bool consecutive = true;
+    for (uint32_t b = 0; b < nb && consecutive; ++b)
+      for (uint32_t i = 1; i < blk_owned[b] && consecutive; ++i)
+        consecutive = cached[blk_cache_off[b] + i] == cached[blk_cache_off[b]] + i;
+    const bool scattered = f.kernel == FOT_KERNEL_GETACC ||
+                           (f.kernel == FOT_KERNEL_MINE && md == 2 && !desc.soa &&
+                            plan_cell.size() >= (1u << 18));
+    if (4 * t > 3 * threads || !(consecutive || scattered)) return FOT_OK;
+  }
   uint64_t owned = 0;
   for (uint32_t n : blk_owned) owned += n;
   std::vector<uint16_t> lists(size_t(owned) * 8, uint16_t(md * cap));
@@ -2874,10 +2895,10 @@ fot_status fot_loop::build_hierarchical() {
   ept = (owner && f.kernel == FOT_KERNEL_RES_CALC && (cfg.flags & FOT_LOOP_TWO_PER_THREAD)) ? 2 : 1;
   threads = std::max<uint32_t>(64, ((max_block + ept - 1) / ept + 63) / 64 * 64);
   if (threads > 1024) return fail(FOT_ERR_UNSUPPORTED, "blocks above 1024 cells");
-  if (may_gather && !owner && !dep_order &&
+  if (!owner && !dep_order &&
       (st = build_gather(blk_cell_off, blk_cache_off, loc, plan_cell)) != FOT_OK)
     return st;
-  if (may_gather && owner &&
+  if (gather_policy != Gather::kNever && owner &&
       (st = build_owner_gather(blk_cell_off, blk_cache_off, blk_owned, cached, loc, colour,
                                         plan_cell)) != FOT_OK)
     return st;
@@ -3144,7 +3165,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
 
 static fot_status fot_loop_create_impl(const fot_functor *f, const fot_problem_desc *desc,
                                       const fot_loop_config *cfg, fot_loop **out,
-                                      bool may_gather = true) {
+                                      fot_loop::Gather policy = fot_loop::Gather::kByRule) {
   if (!f || !desc || !cfg || !out) return fail(FOT_ERR_INVALID_ARGUMENT, "null argument");
   *out = nullptr;
   if (desc->num_mappings == 0 || desc->num_mappings > FOT_MAX_MAPPINGS ||
@@ -3226,7 +3247,7 @@ static fot_status fot_loop_create_impl(const fot_functor *f, const fot_problem_d
   L->base.out = desc->point_data_out;
   L->base.num_cells = desc->num_cells;
   L->base.cell_stride = desc->num_cells;
-  L->may_gather = may_gather;
+  L->gather_policy = policy;
   L->stats.strategy = cfg->strategy;
   L->stats.block_size = cfg->block_size;
   fot_status st;
@@ -3477,7 +3498,10 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
     c.flags = (c.flags & FOT_LOOP_POINT_PARTITION) | FOT_LOOP_OWNER_COMPUTE;
     c.use_graph = 0;
     fot_loop *l = nullptr;
-    if ((st = fot_loop_create_impl(f, &descs[i], &c, &l, gather)) != FOT_OK) return st;
+    if ((st = fot_loop_create_impl(f, &descs[i], &c, &l, gather ? fot_loop::Gather::kAlways
+                                                                : fot_loop::Gather::kNever)) !=
+        FOT_OK)
+      return st;
     B->loops.push_back(l);
     if (gather && !l->gather && l->colour_blk_off.back() > 0) {
       // one kernel runs every problem: plan them all for the colour loop

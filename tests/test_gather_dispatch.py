@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import oracle as O
-from cuda_fot_amd import Problem, capi, meshgen, mini_aero_problem, plan, volna_problem
+from cuda_fot_amd import (Problem, capi, getacc_problem, meshgen, mini_aero_problem, plan,
+                          volna_problem)
 from helpers import airfoil_problem, assert_bitwise, mine_problem, oracle_of
 
 TP = capi.LOOP_TWO_PHASE
@@ -99,3 +100,73 @@ def test_large_soa_plans_of_few_increments_per_point(gpu):
     p.reorder("gps")
     h = check(p, O.VOLNA, capi.functor(capi.KERNEL_VOLNA), 128, 1, True)
     assert h["blocks"] <= 1024
+
+
+# ---- owner compute -----------------------------------------------------------
+def owner_lds(p, op, gather):
+    """LDS of the loop of its own on this plan (gathered sums or colour loop)."""
+    md, td = p.maps[0].shape[1], p.point_data[0].shape[0 if p.soa else 1]
+    if not gather:
+        return (8 * td + 4) * int(op["blk_owned"].max())
+    cap = int(np.diff(op["blk_cell_off"]).max())
+    return 8 * (min(td, 2) if md == 2 else 1) * (md * cap + 1)
+
+
+def owner_gathers(p, kernel, op):
+    md, cells, owned = p.maps[0].shape[1], np.diff(op["blk_cell_off"]), op["blk_owned"]
+    threads = max(64, -(-int(cells.max()) // 64) * 64)
+    half = max(64, -(-max(-(-int(cells.max()) // 2), int(owned.max())) // 64) * 64)
+    consecutive = all(np.all(np.diff(op["cached"][c:c + n].astype(np.int64)) == 1)
+                      for c, n in zip(op["blk_cache_off"], owned))
+    scattered = kernel == O.GETACC or (kernel == O.MINE2 and not p.soa and
+                                       op["cells"].size >= 1 << 18)
+    return 4 * half <= 3 * threads and (consecutive or scattered)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("kind,parts,gather", [
+    ("mine", "points", True), ("mine", "gps", False), ("mine large", "gps", None),
+    ("volna", "points", True), ("volna", "gps", False), ("getacc", "points", True),
+    ("getacc", "gps", True), ("mine4", "points", True), ("mine4", "gps", False),
+    ("mine4", "kway", False), ("getacc", "kway", False)])
+def test_owner_blocks_gather_where_it_is_faster(gpu, kind, parts, gather, soa):
+    """Owner-compute loops on parts with consecutive ids, on GPS-ordered meshes
+    and on k-way cell parts: the kernel planned, and the replay's bits."""
+    md, bs = (4 if kind in ("mine4", "getacc") else 2), 256
+    if kind == "volna":
+        p, kernel = volna_problem(meshgen.tri_mesh(40, 33, seed=1), soa=soa), O.VOLNA
+        f = capi.functor(capi.KERNEL_VOLNA)
+    elif kind == "getacc":
+        p, kernel, f = getacc_problem(61, 83, soa=soa), O.GETACC, capi.functor(capi.KERNEL_GETACC)
+    elif kind == "mine4":
+        cells = meshgen.quad_grid(70, 66)
+        n = 70 * 66
+        pd = meshgen.uniform(4 * n, 1).reshape(n, 4)
+        p = Problem([cells[meshgen.permutation(cells.shape[0], 3)]], [n],
+                    [pd.T.copy() if soa else pd], [meshgen.uniform(4 * cells.shape[0], 2).reshape(4, -1)],
+                    bs, soa)
+        kernel, f = O.MINE4, capi.functor(capi.KERNEL_MINE, 4, 4, 4)
+    else:
+        p = mine_problem(420, 330, soa=soa) if "large" in kind else mine_problem(70, 66, soa=soa)
+        kernel, f = O.MINE2, capi.functor(capi.KERNEL_MINE, 2, 4, 4)
+    p.block_size = bs
+    part = point_part = None
+    if parts == "points":
+        p.partition_points(bs)
+        point_part = p.point_partition
+    elif parts == "gps":
+        p.reorder("gps")
+    else:
+        p.partition(method="kway")
+        p.reorder_to_partition()
+        p.renumber_points()
+        part = p.partition_vector
+    op = plan.owner_plan(p.maps[0], p.num_points[0], bs, part, point_part)
+    want = owner_gathers(p, kernel, op)
+    assert want == (not soa if gather is None else gather)
+    o = oracle_of(p, kernel)
+    O.loop_owner_replay(o, op, 2)
+    stats = p.gpu_loop(f, capi.STRATEGY_HIERARCHICAL, 2, block_size=bs, flags=capi.LOOP_OWNER_COMPUTE)
+    assert stats["lds_bytes"] == owner_lds(p, op, want), stats
+    assert_bitwise(p.point_data[0], o.target, f"{kind} {parts}")
