@@ -1992,9 +1992,17 @@ struct fot_loop {
   uint32_t lds_bytes = 0, threads = 0;
   bool staged = false;
   uint32_t gather_rounds = 1;
-  // whether owner blocks gather: as their rule says, or (a batch's problems)
-  // wherever the kernel takes them, or not at all
-  enum class Gather { kByRule, kAlways, kNever } gather_policy = Gather::kByRule;
+  // whether owner blocks gather: as their rule says, or wherever the kernel takes
+  // them (a batch's problems)
+  enum class Gather { kByRule, kAlways } gather_policy = Gather::kByRule;
+  // what the colour loop needs of an owner plan that gathers, kept on the host
+  // for a batch until every problem's plan is known
+  struct ColourLoop {
+    std::vector<uint16_t> loc;
+    std::vector<uint8_t> colour, blk_ncol;
+    const uint32_t *cached = nullptr;
+    uint32_t threads = 0, lds_bytes = 0;
+  } colour_loop;
   bool gather = false;   // hierarchical: points gather their increments (eng_gather_kernel)
   bool stage_pd = false; // generic hierarchical: the functor's staged input in LDS
   bool dep_order = false;
@@ -2139,6 +2147,8 @@ struct fot_loop {
                           const std::vector<uint32_t> &blk_cache_off,
                           const std::vector<uint16_t> &loc,
                           const std::vector<uint32_t> &plan_cell);
+  // sets the plan up for the colour loop, with the arrays kept in colour_loop
+  fot_status upload_colour_loop();
   fot_status build_atomic();
   fot_status build_global_colour();
   fot_status build_hierarchical();
@@ -2490,6 +2500,25 @@ fot_status fot_loop::build_owner_gather(
   threads = t;
   lds_bytes = lds;
   gather = true;
+  return FOT_OK;
+}
+
+fot_status fot_loop::upload_colour_loop() {
+  fot_status st;
+  uint16_t *d16 = nullptr;
+  uint8_t *d8 = nullptr;
+  const ColourLoop c = std::move(colour_loop);
+  colour_loop = ColourLoop{};
+  if ((st = upload(c.loc.data(), c.loc.size(), &d16)) != FOT_OK) return st;
+  hier.loc = d16;
+  if ((st = upload(c.colour.data(), c.colour.size(), &d8)) != FOT_OK) return st;
+  hier.colour = d8;
+  if ((st = upload(c.blk_ncol.data(), c.blk_ncol.size(), &d8)) != FOT_OK) return st;
+  hier.blk_ncol = d8;
+  hier.cached = c.cached;
+  threads = c.threads;
+  lds_bytes = c.lds_bytes;
+  gather = false;
   return FOT_OK;
 }
 
@@ -2898,18 +2927,19 @@ fot_status fot_loop::build_hierarchical() {
   if (!owner && !dep_order &&
       (st = build_gather(blk_cell_off, blk_cache_off, loc, plan_cell)) != FOT_OK)
     return st;
-  if (gather_policy != Gather::kNever && owner &&
+  colour_loop.cached = hier.cached;
+  colour_loop.threads = threads;
+  colour_loop.lds_bytes = lds_bytes;
+  if (owner &&
       (st = build_owner_gather(blk_cell_off, blk_cache_off, blk_owned, cached, loc, colour,
                                         plan_cell)) != FOT_OK)
     return st;
-  if (!gather) {
-    if ((st = upload(loc.data(), loc.size(), &d16)) != FOT_OK) return st;
-    hier.loc = d16;
-    if ((st = upload(colour.data(), colour.size(), &d8)) != FOT_OK) return st;
-    hier.colour = d8;
-    if ((st = upload(blk_ncol.data(), blk_ncol.size(), &d8)) != FOT_OK) return st;
-    hier.blk_ncol = d8;
+  if (!gather || gather_policy == Gather::kAlways) {
+    colour_loop.loc = std::move(loc);
+    colour_loop.colour = std::move(colour);
+    colour_loop.blk_ncol = blk_ncol;
   }
+  if (!gather && (st = upload_colour_loop()) != FOT_OK) return st;
   if (owner && f.kernel == FOT_KERNEL_RES_CALC) {
     // the staging rounds cover max(cached, nodes) of every block
     uint32_t most = max_nodes;
@@ -3498,18 +3528,15 @@ static fot_status fot_batch_create_impl(const fot_functor *f, uint32_t num_probl
     c.flags = (c.flags & FOT_LOOP_POINT_PARTITION) | FOT_LOOP_OWNER_COMPUTE;
     c.use_graph = 0;
     fot_loop *l = nullptr;
-    if ((st = fot_loop_create_impl(f, &descs[i], &c, &l, gather ? fot_loop::Gather::kAlways
-                                                                : fot_loop::Gather::kNever)) !=
-        FOT_OK)
+    if ((st = fot_loop_create_impl(f, &descs[i], &c, &l, fot_loop::Gather::kAlways)) != FOT_OK)
       return st;
     B->loops.push_back(l);
-    if (gather && !l->gather && l->colour_blk_off.back() > 0) {
-      // one kernel runs every problem: plan them all for the colour loop
-      gather = false;
-      for (fot_loop *p : B->loops) delete p;
-      B->loops.clear();
-      i = 0xffffffffu;
-    }
+    gather = gather && (l->gather || l->colour_blk_off.back() == 0);
+  }
+  // one kernel runs every problem: the colour loop unless all of them gather
+  for (fot_loop *l : B->loops) {
+    if (!gather && l->gather && (st = l->upload_colour_loop()) != FOT_OK) return st;
+    l->colour_loop = {};
   }
   for (uint32_t i = 0; i < num_problems; ++i) {
     const fot_loop *l = B->loops[i];
