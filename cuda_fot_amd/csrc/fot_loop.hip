@@ -50,6 +50,11 @@ struct HierDev {
   // when no other block touches the point; partial sums [slot][TD]
   const uint32_t *wslot;
   double *partial;
+};
+
+// ... and of the kernels that gather, which the colour loops' arguments leave out
+// (two-phase steps of a small mesh paid 0.3 us of 7 for the longer ones)
+struct GatherDev : HierDev {
   // gather accumulation (eng_gather_kernel): block records (first cell, cells,
   // first cached entry, cached points) and per cached entry the increments it
   // adds, in order, as 4 or 8 (`wide`) 16-bit places in the block's LDS planes
@@ -92,7 +97,9 @@ struct RunIO {
 // 701x463 airfoil, two-phase with staged inputs, blocks of 256, 19.1, 20.4 and
 // 18.4.
 struct StepIO {};
-FOT_DEV RunIO run_io(double *out, StepIO) { return {out, out, nullptr, nullptr}; }
+__host__ __device__ inline RunIO run_io(double *out, StepIO) {
+  return {out, out, nullptr, nullptr};
+}
 FOT_DEV RunIO run_io(double *, const RunIO &run) { return run; }
 
 // Two-phase writeback of a block's cache entry i (point g, values v): added
@@ -583,7 +590,7 @@ template <class F, bool SOA> struct RowIds {
 // place.
 template <class F, bool SOA, int R, class IO, int LB = 1024, bool NTC = false>
 __global__ __launch_bounds__(LB, LB < 1024 ? kSmallBoundWaves<F> : 1) void eng_gather_kernel(
-    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, HierDev h, IO run,
+    std::conditional_t<NTC, StreamCellArgs, EngineArgs> a, GatherDev h, IO run,
     uint32_t blk_begin, uint32_t nbc) {
   const RunIO io = run_io(a.out, run);
   constexpr uint32_t MD = F::MD, TD = F::TD, PD = std::min(kPassDims<F>, TD);
@@ -832,7 +839,7 @@ __global__ __launch_bounds__(1024) void res_calc_hier_staged_kernel(EngineArgs a
 // the fluxes it adds or, as the edge's second cell, subtracts (place | 0x8000;
 // its increment is -f, and v + (-f) is v - f).
 template <bool SOA, int R, class IO>
-__global__ __launch_bounds__(1024) void res_calc_hier_gather_kernel(EngineArgs a, HierDev h,
+__global__ __launch_bounds__(1024) void res_calc_hier_gather_kernel(EngineArgs a, GatherDev h,
                                                                     IO run, uint32_t blk_begin,
                                                                     uint32_t nbc) {
   const RunIO io = run_io(a.out, run);
@@ -1056,7 +1063,7 @@ template <class F> constexpr uint32_t owner_gather_lds(uint32_t cap) {
 }
 
 template <class F, bool SOA>
-__device__ __forceinline__ void owner_gather_block(const EngineArgs &a, const HierDev &h,
+__device__ __forceinline__ void owner_gather_block(const EngineArgs &a, const GatherDev &h,
                                                    const RunIO &io, const OwnerItem &it,
                                                    double *lds) {
   constexpr uint32_t MD = F::MD, TD = F::TD, PD = kOwnerPassDims<F>;
@@ -1137,7 +1144,7 @@ __device__ __forceinline__ void owner_gather_block(const EngineArgs &a, const Hi
 }
 
 template <class F, bool SOA, class IO>
-__global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, HierDev h,
+__global__ __launch_bounds__(512) void eng_owner_gather_kernel(EngineArgs a, GatherDev h,
                                                                uint32_t nb, IO run) {
   extern __shared__ double lds[];
   owner_gather_block<F, SOA>(a, h, run_io(a.out, run), h.items[xcd_block(blockIdx.x, nb)], lds);
@@ -1153,7 +1160,7 @@ __global__ __launch_bounds__(LB) void eng_owner_kernel(EngineArgs a, HierDev h, 
 // One problem of a batch: its engine arguments and owner-compute plan.
 struct BatchProblem {
   EngineArgs args;
-  HierDev hier;
+  GatherDev hier;
 };
 
 // A pointer read from memory, as one to global memory.  The compiler takes
@@ -1172,7 +1179,7 @@ FOT_DEV BatchProblem as_global(const BatchProblem &from) {
   for (uint32_t k = 0; k < FOT_MAX_CELL_DATA; ++k)
     p.args.cell_data[k] = as_global(p.args.cell_data[k]);
   p.args.out = as_global(p.args.out);
-  HierDev &h = p.hier;
+  GatherDev &h = p.hier;
   h.blk_cell_off = as_global(h.blk_cell_off), h.blk_cache_off = as_global(h.blk_cache_off);
   h.blk_owned = as_global(h.blk_owned), h.blk_ncol = as_global(h.blk_ncol);
   h.cached = as_global(h.cached), h.loc = as_global(h.loc), h.colour = as_global(h.colour);
@@ -1781,16 +1788,19 @@ __global__ __launch_bounds__(1024) void res_calc_owner4_kernel(EngineArgs a,
 }
 
 // the gather kernel instantiation for a plan: one block per workgroup or
-// persistent, edges per thread, staging rounds, list words, owned rounds
+// persistent, edges per thread, staging rounds, list words, owned rounds.  IO:
+// the forms that only an option asks for (persistent, per-cell terms, lists from
+// the plan) run their plain steps on the run's kernel, to keep the library small.
 template <bool SOA, int E, int K, int W, int O, class IO>
 const void *owner3_pick(bool persistent, bool pre) {
+  if (persistent)
+    return pre ? reinterpret_cast<const void *>(
+                     &res_calc_owner4_kernel<SOA, E, K, W, O, true, RunIO>)
+               : reinterpret_cast<const void *>(
+                     &res_calc_owner4_kernel<SOA, E, K, W, O, false, RunIO>);
   if (pre)
-    return persistent
-               ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, true, IO>)
-               : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, true, IO>);
-  return persistent
-             ? reinterpret_cast<const void *>(&res_calc_owner4_kernel<SOA, E, K, W, O, false, IO>)
-             : reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, false, IO>);
+    return reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, true, RunIO>);
+  return reinterpret_cast<const void *>(&res_calc_owner3_kernel<SOA, E, K, W, O, false, IO>);
 }
 template <bool SOA, int E, int K, class IO>
 const void *owner3_pick_w(bool persistent, bool pre, uint32_t lw, bool ko1, bool nt) {
@@ -1801,10 +1811,10 @@ const void *owner3_pick_w(bool persistent, bool pre, uint32_t lw, bool ko1, bool
     return ko1 ? owner3_pick<SOA, E, K, 0, 1, IO>(persistent, pre)
                : owner3_pick<SOA, E, K, 0, K, IO>(persistent, pre);
   if (lw == 2)
-    return ko1 ? owner3_pick<SOA, E, K, 2, 1, IO>(persistent, pre)
-               : owner3_pick<SOA, E, K, 2, K, IO>(persistent, pre);
-  return ko1 ? owner3_pick<SOA, E, K, 4, 1, IO>(persistent, pre)
-             : owner3_pick<SOA, E, K, 4, K, IO>(persistent, pre);
+    return ko1 ? owner3_pick<SOA, E, K, 2, 1, RunIO>(persistent, pre)
+               : owner3_pick<SOA, E, K, 2, K, RunIO>(persistent, pre);
+  return ko1 ? owner3_pick<SOA, E, K, 4, 1, RunIO>(persistent, pre)
+             : owner3_pick<SOA, E, K, 4, K, RunIO>(persistent, pre);
 }
 template <bool SOA, int E, class IO>
 const void *owner3_pick_k(bool persistent, bool pre, uint32_t ks, uint32_t lw, bool ko1,
@@ -1913,7 +1923,7 @@ void launch_eng_hier(bool stage, uint32_t grid, uint32_t threads, uint32_t lds, 
 // Launches eng_owner_gather_kernel or eng_owner_kernel; IO: StepIO or RunIO.
 template <class F, bool SOA, class IO>
 void launch_owner(bool gather, uint32_t nb, uint32_t threads, uint32_t lds, hipStream_t s,
-                  const EngineArgs &a, const HierDev &h, const IO &io) {
+                  const EngineArgs &a, const GatherDev &h, const IO &io) {
   constexpr int SB = kSmallBound<F>;
   if constexpr (kOwnerGathers<F>) {
     if (gather) {
@@ -1933,7 +1943,7 @@ void launch_owner(bool gather, uint32_t nb, uint32_t threads, uint32_t lds, hipS
 // Launches eng_gather_kernel<F, SOA, R>.
 template <class F, bool SOA, int R, class IO>
 void launch_gather(uint32_t grid, uint32_t threads, uint32_t lds, hipStream_t s,
-                   const EngineArgs &a, const HierDev &h, const IO &io, uint32_t b0,
+                   const EngineArgs &a, const GatherDev &h, const IO &io, uint32_t b0,
                    uint32_t nbc, bool stream_cells) {
   constexpr int SB = kSmallBound<F>;
   const bool small = threads <= uint32_t(SB);
@@ -1986,7 +1996,7 @@ struct fot_loop {
   // global colour
   std::vector<EngineArgs> colour_args;
   // hierarchical
-  HierDev hier{};
+  GatherDev hier{};
   EngineArgs plan_args{};
   std::vector<uint32_t> colour_blk_off;
   uint32_t lds_bytes = 0, threads = 0;
@@ -3114,7 +3124,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
           const OwnerMeta *om = owner_meta;
           const uint32_t *pc = hier.cached, *pp = hier.packed, *pl = owner_plist;
           uint32_t nbv = nb;
-          RunIO iov = run ? *run : RunIO{}; // (a StepIO takes its first byte)
+          RunIO iov = run ? *run : run_io(base.out, StepIO{}); // (or a StepIO's byte)
           void *kargs[] = {&pa, &om, &pc, &pp, &pl, &nbv, &iov};
           FOT_HIP(hipLaunchKernel(run ? owner3_run_fn : owner3_fn, dim3(launch_grid),
                                   dim3(threads), kargs, size_t(lds_bytes), s));
