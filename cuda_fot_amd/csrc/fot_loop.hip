@@ -189,7 +189,8 @@ FOT_DEV void load_loc(const uint16_t *__restrict__ p, uint32_t *loc) {
 // here, one per lane's row or value: one atomic per increment 359 us on the
 // GPS-ordered 1200x600 airfoil (SOA 267), whole rows by consecutive lanes but
 // unmerged 93, merged here 40 (SOA 40); shuffled 518 -> 206; mine 1024^2 on
-// compact blocks 559 -> 57, hex 64^3 255 -> 34.
+// compact blocks 559 -> 57, hex 64^3 255 -> 34.  Small meshes of cells with many
+// points have too few requests for that: see direct_atomics.
 template <uint32_t TD> struct PointTable {
   static constexpr uint32_t kBytesPerSlot = TD * 8 + 4;
   // probes before an increment goes to memory by itself (a full table: a
@@ -252,7 +253,7 @@ template <uint32_t TD> struct PointTable {
   }
 };
 
-template <class F, bool SOA, int LB = 1024>
+template <class F, bool SOA, bool ATOMIC, int LB = 1024>
 __global__ __launch_bounds__(LB) void eng_direct_kernel(EngineArgs a) {
   const uint32_t ind = blockIdx.x * blockDim.x + threadIdx.x;
   if (ind >= a.num_cells) return;
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(LB) void eng_direct_kernel(EngineArgs a) {
   double inc[F::MD * F::TD];
   targets<F>(a, ind, tgt);
   F::template compute<SOA>(a, ind, tgt, inc);
-  add_increments<F, SOA, false>(a.out, a.num_points[0], tgt, inc);
+  add_increments<F, SOA, ATOMIC>(a.out, a.num_points[0], tgt, inc);
 }
 
 template <class F, bool SOA, int LB = 1024>
@@ -2001,6 +2002,7 @@ struct fot_loop {
   std::vector<uint32_t> colour_blk_off;
   uint32_t lds_bytes = 0, threads = 0;
   bool staged = false;
+  bool ordered = false; // atomics: consecutive cells share points (direct_atomics)
   uint32_t gather_rounds = 1;
   // whether owner blocks gather: as their rule says, or wherever the kernel takes
   // them (a batch's problems)
@@ -2185,6 +2187,20 @@ fot_status fot_loop::build_atomic() {
     fot_status st = upload(desc.cell_to_node[m], size_t(desc.num_cells) * desc.mesh_dim[m], &d);
     if (st != FOT_OK) return st;
     base.maps[m] = d;
+  }
+  // whether consecutive cells share points, where direct_atomics asks
+  const uint32_t md = desc.mesh_dim[0];
+  if (md >= 4 && uint64_t(md) * desc.num_cells < 600000) {
+    constexpr uint32_t kRun = 64;
+    std::vector<uint32_t> ids;
+    uint64_t distinct = 0;
+    for (size_t c = 0; c < desc.num_cells; c += kRun) {
+      const size_t n = std::min<size_t>(kRun, desc.num_cells - c);
+      ids.assign(desc.cell_to_node[0] + c * md, desc.cell_to_node[0] + (c + n) * md);
+      std::sort(ids.begin(), ids.end());
+      distinct += uint64_t(std::unique(ids.begin(), ids.end()) - ids.begin());
+    }
+    ordered = 2 * uint64_t(md) * desc.num_cells >= 3 * distinct;
   }
   stats.num_launches_per_iter = 1;
   return FOT_OK;
@@ -3040,19 +3056,46 @@ fot_status fot_loop::build_hierarchical() {
   return FOT_OK;
 }
 
-// Threads of an atomics workgroup.  Larger ones merge more increments of one
-// point before they reach memory: 1200x600 airfoil, GPS-ordered, 128 / 256 /
-// 512 / 1024 threads 59 / 94 / 40 / 42 us (256 fill their table, the next
-// power of two, to the brim).  Meshes too small to fill the chip that way run
-// 128, by their increments (edges of two cells, 9 000 to 90 000: 3.7-5.0 us
-// against 4.3-5.1 with 512; 160 000: 8.6 against 6.7; lulesh 48^3, 110 000
-// elements of eight nodes: 31 against 21), mini_aero's registers ask for 256
-// (48^3: 34 us against 42), and the table has to fit the LDS.
+// Threads of a workgroup of the atomics loop's table.  Larger ones merge more
+// increments of one point before they reach memory: 1200x600 airfoil,
+// GPS-ordered, 128 / 256 / 512 / 1024 threads 59 / 94 / 40 / 42 us (a workgroup's
+// points are two runs of ids a level of the ordering, some 600, apart; modulo 512
+// slots they coincide: counted on the host 3.5 probes per point and 75 of 512
+// increments past the table, with 256 slots 1.7 and 16 of 256, with 1024 and more
+// none).  Meshes too small to fill the chip that way run 128, by their increments
+// (edges of two cells, 9 000 to 90 000: 3.7-5.0 us against 4.3-5.1 with 512;
+// 160 000: 8.6 against 6.7; lulesh 48^3, 110 000 elements of eight nodes: 31
+// against 21), mini_aero's registers ask for 256 (48^3: 34 us against 42), and the
+// table has to fit the LDS.
 template <class F> uint32_t atomic_threads(uint32_t cells) {
   uint32_t n = uint64_t(F::MD) * cells < (1u << 18) ? 128u : kSmallBound<F> < 1024 ? 256u : 512u;
   while (PointTable<F::TD>::slots_for(F::MD * n) * PointTable<F::TD>::kBytesPerSlot > 144u * 1024u)
     n /= 2;
   return n;
+}
+
+// Whether the atomics loop adds every increment by itself: on small ordered
+// meshes of cells with four or eight points the atomics spread over the L2s, and
+// the table's probes are a chain of their own.  n: increments; ordered: runs of 64
+// cells add at least 1.5 increments per point they name (on a shuffled mesh the
+// table adds whole rows where single values would go, and is faster at any size).
+// Time by itself over time in the table, GPS-ordered:
+//   hex and lulesh (8 points, 3 values): 17 600 increments 0.84, 74 000 0.80, 175 000
+//     1.43; SOA 74 000 0.56, 175 000 0.86, 262 000 1.12
+//   mine of 8 points, 1 value: 17 000 1.11, 54 000 0.66, 343 000 0.89 (shuffled 0.95),
+//     551 000 0.84 (1.12), 941 000 1.13; 2 values: 54 000 0.64, 157 000 0.90, 343 000
+//     1.5; 4 values: 27 000 1.09, SOA 111 000 0.83, 195 000 1.07; 8 values: above 1
+//   getacc (4 points, 4 values): 9 600 0.93, 24 000 1.09; SOA 39 000 0.87, 101 000
+//     1.08; mine of 4 points 0.95 to 1.08 there with 4 values, above 1 with others
+//   cells of 2 points: above 1, or level at 8 000 and below
+template <class F, bool SOA> constexpr bool direct_atomics(uint64_t n, bool ordered) {
+  if (F::MD >= 8) {
+    if (F::TD == 1) return n >= 20000 && n < (ordered ? 600000 : 350000);
+    if (F::TD == 2) return ordered && n >= 20000 && n < 200000;
+    if (F::TD == 3) return ordered && n < (SOA ? 200000 : 100000);
+    return ordered && F::TD == 4 && SOA && n < 150000;
+  }
+  return ordered && F::MD >= 4 && F::TD == 4 && n < (SOA ? 48000 : 20000);
 }
 
 template <class F, bool SOA, class IO, class Colours>
@@ -3083,7 +3126,11 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
     // direct launches: one thread per cell, whatever the block size
     constexpr int LB = kSmallBound<F>;
     const uint32_t dbs = std::min<uint32_t>(bs, LB);
-    if (cfg.strategy == FOT_STRATEGY_ATOMIC) {
+    if (cfg.strategy == FOT_STRATEGY_ATOMIC &&
+        direct_atomics<F, SOA>(uint64_t(F::MD) * desc.num_cells, ordered)) {
+      hipLaunchKernelGGL((eng_direct_kernel<F, SOA, true, LB>),
+                         dim3((desc.num_cells + dbs - 1) / dbs), dim3(dbs), 0, s, base);
+    } else if (cfg.strategy == FOT_STRATEGY_ATOMIC) {
       const uint32_t at = atomic_threads<F>(desc.num_cells);
       const uint32_t slots = PointTable<F::TD>::slots_for(F::MD * at);
       const uint32_t lds = slots * PointTable<F::TD>::kBytesPerSlot;
@@ -3095,7 +3142,7 @@ fot_status fot_loop::enqueue(hipStream_t s, const RunIO *run) {
     } else if (cfg.strategy == FOT_STRATEGY_GLOBAL_COLOUR) {
       for (const EngineArgs &a : colour_args) {
         if (a.num_cells == 0) continue;
-        hipLaunchKernelGGL((eng_direct_kernel<F, SOA, LB>),
+        hipLaunchKernelGGL((eng_direct_kernel<F, SOA, false, LB>),
                            dim3((a.num_cells + dbs - 1) / dbs), dim3(dbs), 0, s, a);
       }
     } else if (owner) {

@@ -480,8 +480,9 @@ typedef struct {
 
 typedef struct {
   uint32_t strategy;      /* fot_strategy */
-  uint32_t block_size;    /* threads (global colour) or cells per block; the
-                             atomics loop sizes its own workgroups */
+  uint32_t block_size;    /* threads (global colour, atomics of small ordered
+                             meshes) or cells per block; other atomics loops
+                             size their own workgroups */
   const uint32_t *partition; /* HOST, nullable: block id per cell */
   uint32_t use_graph;     /* capture one iteration in a hipGraph */
   uint32_t flags;         /* FOT_LOOP_* */

@@ -7,7 +7,8 @@ import pytest
 import oracle as O
 from cuda_fot_amd import (Problem, capi, getacc_problem, meshgen, mini_aero_problem, plan,
                           volna_problem)
-from helpers import airfoil_problem, assert_bitwise, mine_problem, oracle_of
+from helpers import (airfoil_problem, assert_bitwise, assert_close_scaled, mine_problem,
+                     oracle_of)
 
 TP = capi.LOOP_TWO_PHASE
 STAGED_DIM = {O.MINI_AERO: 28, O.LULESH: 3}
@@ -170,3 +171,35 @@ def test_owner_blocks_gather_where_it_is_faster(gpu, kind, parts, gather, soa):
     stats = p.gpu_loop(f, capi.STRATEGY_HIERARCHICAL, 2, block_size=bs, flags=capi.LOOP_OWNER_COMPUTE)
     assert stats["lds_bytes"] == owner_lds(p, op, want), stats
     assert_bitwise(p.point_data[0], o.target, f"{kind} {parts}")
+
+
+# ---- atomics -------------------------------------------------------------------
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("order", [None, "gps"])
+@pytest.mark.parametrize("kind,n", [("hex", 12), ("hex", 24), ("hex", 30), ("getacc", 50),
+                                    ("getacc", 112), ("mine8", 14), ("mine8", 27), ("mine8", 43)])
+def test_atomics_by_themselves_and_in_the_table(gpu, kind, n, order, soa):
+    """The atomics loop on either side of the sizes where small meshes of cells
+    with four or eight points leave the table out, ordered and shuffled."""
+    points = n + 1
+    if kind == "getacc":
+        p, kernel, f = getacc_problem(points, points, soa=soa), O.GETACC, \
+            capi.functor(capi.KERNEL_GETACC)
+    else:
+        cells = meshgen.hex_grid(points, points, points)
+        cells = cells[meshgen.permutation(cells.shape[0], 3)]
+        td = 3 if kind == "hex" else 4
+        pd = meshgen.uniform(td * points ** 3, 1).reshape(-1, td)
+        data = meshgen.normal(cells.shape[0] * (24 if kind == "hex" else 4), 2)
+        p = Problem([cells], [points ** 3], [pd.T.copy() if soa else pd],
+                    [data.reshape(-1, cells.shape[0])], 128, soa)
+        kernel = O.HEX_SCATTER if kind == "hex" else O.MINE8
+        f = capi.functor(capi.KERNEL_HEX_SCATTER) if kind == "hex" else \
+            capi.functor(capi.KERNEL_MINE, 8, 4, 4)
+    if order:
+        p.reorder(order)
+    o = oracle_of(p, kernel)
+    scale = o.loop_serial(1, with_scale=True)
+    p.gpu_loop(f, capi.STRATEGY_ATOMIC, 1, block_size=96)
+    assert_close_scaled(p.point_data[0], o.target, scale, what=f"{kind} {n}")
