@@ -2144,8 +2144,7 @@ struct fot_loop {
     return FOT_OK;
   }
 
-  // the plan of eng_gather_kernel, when the blocks allow it: sets `gather`
-  // the same for owner_gather_block
+  // the plan of owner_gather_block, when the blocks allow it: sets `gather`
   fot_status build_owner_gather(const std::vector<uint32_t> &blk_cell_off,
                                 const std::vector<uint32_t> &blk_cache_off,
                                 const std::vector<uint32_t> &blk_owned,
@@ -2155,6 +2154,7 @@ struct fot_loop {
                                 const std::vector<uint32_t> &plan_cell);
   std::vector<OwnerItem> owner_items;
   uint32_t most_cells = 0, most_owned = 0;
+  // the same for eng_gather_kernel and res_calc_hier_gather_kernel
   fot_status build_gather(const std::vector<uint32_t> &blk_cell_off,
                           const std::vector<uint32_t> &blk_cache_off,
                           const std::vector<uint16_t> &loc,
@@ -2358,8 +2358,9 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
     const double per_point = double(loc.size()) / blk_cache_off[nb];
     if (desc.soa ? two_phase && nb > 1024 && per_point < 1.6 : per_point < 2.4) return FOT_OK;
   }
-  // res_calc_hier_gather_kernel, where the plan's blocks do not fill the chip
-  // for one round and their latency is what counts (colour loop / this, a
+  // res_calc_hier_gather_kernel, where the plan's blocks (of all colours
+  // together: where the line was measured, not what one launch of a per-colour
+  // step holds) are few and their latency is what counts (colour loop / this, a
   // step: 64x32 8.9 / 7.2 us, 200x150 10.0 / 7.6, blocks of 512; 701x463,
   // blocks of 1024, 20.6 / 18.1); beyond that its registers and LDS traffic
   // cost as much as they save (701x463, blocks of 512, SOA 25.0 / 25.0;

@@ -1,14 +1,16 @@
 """Which hierarchical plans gather their sums, and that either kernel gives the
 oracle's bits.  The rule is restated here on the host plan; the loop's LDS size
 tells which kernel was planned."""
+import copy
+
 import numpy as np
 import pytest
 
 import oracle as O
-from cuda_fot_amd import (Problem, capi, getacc_problem, meshgen, mini_aero_problem, plan,
-                          volna_problem)
-from helpers import (airfoil_problem, assert_bitwise, assert_close_scaled, mine_problem,
-                     oracle_of)
+from cuda_fot_amd import (Problem, capi, getacc_problem, lulesh_problem, meshgen,
+                          mini_aero_problem, plan, volna_problem)
+from helpers import (airfoil_problem, assert_bitwise, assert_close_scaled, hex_problem,
+                     mine_problem, oracle_of)
 
 TP = capi.LOOP_TWO_PHASE
 STAGED_DIM = {O.MINI_AERO: 28, O.LULESH: 3}
@@ -203,3 +205,125 @@ def test_atomics_by_themselves_and_in_the_table(gpu, kind, n, order, soa):
     scale = o.loop_serial(1, with_scale=True)
     p.gpu_loop(f, capi.STRATEGY_ATOMIC, 1, block_size=96)
     assert_close_scaled(p.point_data[0], o.target, scale, what=f"{kind} {n}")
+
+
+# ---- the gathering kernels of each functor --------------------------------------
+NT = capi.LOOP_NONTEMPORAL
+STAGE = capi.LOOP_STAGE_INPUTS
+
+
+def element_problem(kind, n, soa):
+    if kind == "lulesh":
+        return lulesh_problem(n + 1, n, n + 2, soa=soa), O.LULESH, capi.functor(capi.KERNEL_LULESH)
+    if kind == "getacc":
+        return getacc_problem(5 * n, 4 * n, soa=soa), O.GETACC, capi.functor(capi.KERNEL_GETACC)
+    return hex_problem(n, soa=soa), O.HEX_SCATTER, capi.functor(capi.KERNEL_HEX_SCATTER)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("kind,n,method,block_size,gather", [
+    ("hex", 13, "bisect", 256, True), ("hex", 13, "bisect", 128, False),
+    ("hex", 9, None, 128, False), ("lulesh", 13, "bisect", 512, True),
+    ("lulesh", 13, "bisect", 256, True), ("lulesh", 13, None, 256, False),
+    ("getacc", 12, "bisect", 128, True), ("getacc", 12, "bisect", 512, True),
+    ("getacc", 14, None, 256, False)])
+def test_element_loops_gather_on_compact_parts(gpu, kind, n, method, block_size, gather, soa):
+    """hex, lulesh and getacc on parts that gather and on blocks with too many
+    points that do not: per colour, two-phase and with nontemporal cell data,
+    bits of the oracle's replay; lulesh's volumes come from either kernel."""
+    p, kernel, f = element_problem(kind, n, soa)
+    p.block_size = block_size
+    if method:
+        p.partition(method=method)
+        p.reorder_to_partition()
+        p.renumber_points()
+    flags = (0, TP, TP | NT) if kind != "getacc" else (0, TP)
+    volumes = None
+    if kind == "lulesh":
+        o = oracle_of(p, kernel)
+        o.loop_serial(1)
+        volumes = np.array(o.cell_data[1])
+    for iters in (1, 2):
+        q = copy.deepcopy(p)
+        for fl in flags:
+            check(q, kernel, f, block_size, iters, gather, (fl,))
+            if volumes is not None:
+                assert_bitwise(q.cell_data[1], volumes, f"volumes, flags {fl}")
+                q.cell_data[1][:] = np.nan
+            q.point_data = copy.deepcopy(p.point_data)
+
+
+# ---- lists of exactly 4, 8 and 9 increments in a block ---------------------------
+def hub_blocks(degree, blocks=5):
+    """Edges in blocks of 64, every block a bipartite graph of its own first points
+    and of second points it shares with its neighbour, whose first points have
+    `degree` edges; (edges, points)."""
+    per = 64 // degree                    # first points a block
+    edges = []
+    for b in range(blocks):
+        first = np.repeat(np.arange(per), degree)
+        second = (first + np.tile(np.arange(degree), per)) % max(per, degree)
+        e = np.stack([32 * b + first, 1000 + 40 * (b // 2) + second], 1)
+        rest = 64 - e.shape[0]            # (degree 9: one more edge of two points more)
+        extra = np.stack([32 * b + 20 + np.arange(rest), 1000 + 40 * (b // 2) + 30 + np.arange(rest)], 1)
+        block = np.concatenate([e, extra])
+        edges.append(block[np.random.default_rng(b).permutation(64)])
+    edges = np.concatenate(edges)
+    ids, at = np.unique(edges, return_inverse=True)
+    return at.reshape(edges.shape).astype(np.uint32), ids.size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("degree", [4, 8, 9])
+def test_hierarchical_lists_of_4_8_and_9(gpu, degree, soa):
+    maps, n = hub_blocks(degree)
+    pd = meshgen.uniform(4 * n, 1).reshape(n, 4)
+    p = Problem([maps], [n], [pd.T.copy() if soa else pd],
+                [meshgen.uniform(4 * maps.shape[0], 2).reshape(4, -1)], 64, soa)
+    h = check(p, O.MINE2, capi.functor(capi.KERNEL_MINE, 2, 4, 4), 64, 2, degree <= 8)
+    assert h["longest"] == degree and h["threads"] == 64
+
+
+def staged_check(p, gather, block_size, iters=2):
+    """Staged res_calc per colour and two-phase against the replay, on the kernel
+    expected."""
+    h = host_plan(p, block_size)
+    assert gather == (h["blocks"] < 1024 and h["longest"] <= 8 and h["most"] <= 2 * h["threads"])
+    o = oracle_of(p, O.RES_CALC)
+    o.loop_hier_replay(O.OraclePlan(p.maps, p.num_points[0], block_size, p.partition_vector), iters)
+    start = [d.copy() for d in p.point_data]
+    for fl in (STAGE, STAGE | TP):
+        p.point_data = [d.copy() for d in start]
+        stats = p.gpu_loop(capi.functor(capi.KERNEL_RES_CALC), capi.STRATEGY_HIERARCHICAL, iters,
+                           block_size=block_size, flags=fl)
+        lds = 8 * max(5 * h["most"], 4 * (h["threads"] + 1)) if gather else 72 * h["most"]
+        assert stats["lds_bytes"] == lds, (stats, h)
+        assert_bitwise(p.point_data[0], o.target, f"flags {fl} {h}")
+    return h
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("degree", [4, 8, 9])
+def test_staged_res_calc_lists_of_4_8_and_9(gpu, degree, soa):
+    maps, n = hub_blocks(degree)
+    rng = np.random.default_rng(degree)
+    q = np.array([1.0, 0.4, 0.0, 2.5]) * (1 + 1e-2 * rng.normal(size=(n, 4)))
+    res, x, adt = rng.normal(size=(n, 4)), rng.normal(size=(50, 2)), rng.uniform(0.5, 1.5, n)
+    nodes = rng.integers(0, 50, maps.shape).astype(np.uint32)
+    if soa:
+        res, x, q = res.T.copy(), x.T.copy(), q.T.copy()
+    p = Problem([maps, nodes, maps, maps], [n, 50, n, n], [res, x, q, adt], (), 64, soa)
+    assert staged_check(p, degree <= 8, 64)["longest"] == degree
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("nx,ny,gather", [(236, 139, True), (240, 140, False)])
+def test_staged_res_calc_on_either_side_of_1024_blocks(gpu, nx, ny, gather, soa):
+    p = airfoil_problem(nx, ny, soa=soa, res0_seed=4)
+    p.reorder("gps")
+    h = staged_check(p, gather, 64, 1)
+    assert 1000 <= h["blocks"] < 1060

@@ -174,3 +174,56 @@ def test_mlp_loss_of_equal_terms_is_the_term(gpu, rows):
         loss, _ = net.loss_grad(np.ones((rows, 1), np.float32), np.full((rows, 1), value),
                                 None)
         assert np.float32(loss) == value * value
+
+
+def _adam(p, x, t, mask, shape, epochs, lr, decay, state, noise=None):
+    """FP64 Adam on the oracle's gradient; state: moments and steps taken.  noise
+    (a generator): the gradients off by 16 FP32 roundings of the largest."""
+    b1, b2, eps = (float(np.float32(v)) for v in (0.9, 0.999, 1e-8))
+    losses = []
+    for _ in range(epochs):
+        loss, g = MO.loss_grad(p, x, t, mask, *shape)
+        losses.append(loss)
+        if noise is not None:
+            g = g + 16 * 2.0 ** -24 * np.abs(g).max() * noise.standard_normal(g.size)
+        g = g + decay * p
+        state["n"] += 1
+        state["m"] = b1 * state["m"] + (1 - b1) * g
+        state["v"] = b2 * state["v"] + (1 - b2) * g * g
+        rate = lr * np.sqrt(1 - b2 ** state["n"]) / (1 - b1 ** state["n"])
+        p = p - rate * state["m"] / (np.sqrt(state["v"]) + eps)
+    return p, losses
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_in,hidden,n_out,rows,masked", [
+    (24, 64, 6, 95, True), (33, 40, 7, 200, False),  # in two launches
+    (24, 65, 6, 50, True), (65, 16, 3, 50, False)])  # layer by layer
+def test_mlp_training_follows_adam(gpu, n_in, hidden, n_out, rows, masked):
+    """Losses and parameters over two calls of train() against FP64 Adam: within
+    ten times what gradients off by 16 FP32 roundings change in it.  (A decay rate
+    of 0.998 for 0.999 moves the median parameter 50 times as far.)"""
+    from cuda_fot_amd.mlp import MLP
+    rng = np.random.default_rng(rows)
+    net = MLP(n_in, hidden, n_out)
+    net.set_params(rng.normal(0, 0.2, net.num_params).astype(np.float32))
+    p0 = net.get_params().astype(np.float64)
+    x = rng.normal(size=(rows, n_in)).astype(np.float32)
+    t = rng.normal(size=(rows, n_out)).astype(np.float32)
+    m = (rng.random((rows, n_out)) > 0.2).astype(np.float32) if masked else None
+    calls = ((6, float(np.float32(0.02))), (4, float(np.float32(0.01))))
+    decay = float(np.float32(0.1))
+    runs = []
+    for noise in (None, np.random.default_rng(1)):
+        state, p, losses = dict(m=0.0, v=0.0, n=0), p0, []
+        for epochs, lr in calls:
+            p, l = _adam(p, x, t, m, (n_in, hidden, n_out), epochs, lr, decay, state, noise)
+            losses += l
+        runs.append((p, np.array(losses)))
+    (ref, ref_loss), (off, off_loss) = runs
+    losses = np.concatenate([net.train(x, t, m, epochs=e, lr=lr, weight_decay=decay)
+                             for e, lr in calls])
+    assert np.abs(losses / ref_loss - 1).max() <= 10 * np.abs(off_loss / ref_loss - 1).max() + 2e-6
+    err, bound = np.abs(net.get_params() - ref), np.abs(off - ref)
+    assert np.median(err) <= 10 * np.median(bound)
+    assert np.quantile(err, 0.99) <= 10 * np.quantile(bound, 0.99)
