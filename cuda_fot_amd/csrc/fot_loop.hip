@@ -2353,10 +2353,14 @@ fot_status fot_loop::build_gather(const std::vector<uint32_t> &blk_cell_off,
   // level (mini_aero 55^3 in blocks of 256 76.3 / 75.1 per colour), from 2.5 on
   // gathered is faster, by 2 to 20 % on compact parts (2.5 to 3.6).  In SOA it is
   // faster per colour at any ratio (2 to 30 %), and two-phase but for large plans
-  // of the lowest (volna, 1.27 M edges in blocks of 512: 49.9 / 54.1).
+  // of the lowest (volna, 1.27 M edges in blocks of 512: 49.9 / 54.1) and, where
+  // rows are staged, of up to 2.5 (mini_aero 55^3 in blocks of 128 40.6 / 44.2, of
+  // 256 39.4 / 42.2, of 512 level).
   if (md == 2 && !staged && !stage_pd) {
     const double per_point = double(loc.size()) / blk_cache_off[nb];
-    if (desc.soa ? two_phase && nb > 1024 && per_point < 1.6 : per_point < 2.4) return FOT_OK;
+    const bool few = desc.soa ? two_phase && nb > 1024 && per_point < (stages ? 2.5 : 1.6)
+                              : per_point < 2.4;
+    if (few) return FOT_OK;
   }
   // res_calc_hier_gather_kernel, where the plan's blocks (of all colours
   // together: where the line was measured, not what one launch of a per-colour

@@ -37,7 +37,8 @@ def gathers(p, kernel, h, two_phase):
         return False
     if md == 2:
         if p.soa:
-            return not (two_phase and h["blocks"] > 1024 and h["per_point"] < 1.6)
+            low = 2.5 if kernel in STAGED_DIM else 1.6
+            return not (two_phase and h["blocks"] > 1024 and h["per_point"] < low)
         return h["per_point"] >= 2.4
     return True
 
@@ -103,6 +104,10 @@ def test_large_soa_plans_of_few_increments_per_point(gpu):
     p.reorder("gps")
     h = check(p, O.VOLNA, capi.functor(capi.KERNEL_VOLNA), 128, 1, True)
     assert h["blocks"] <= 1024
+    p = mini_aero_problem(meshgen.hex_faces(36, 36, 36), soa=True)
+    p.reorder("gps")
+    h = check(p, O.MINI_AERO, capi.functor(capi.KERNEL_MINI_AERO), 128, 1, (True, False))
+    assert h["blocks"] > 1024 and 2.0 < h["per_point"] < 2.5
 
 
 # ---- owner compute -----------------------------------------------------------
