@@ -146,3 +146,26 @@ def test_owner_res_calc_run_on_an_iterate_of_any_alignment(gpu, aligned):
     if not aligned:
         assert room.download()[0] == 7.0 and room.download()[n + 1] == 9.0
     loop.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("stage", [0, capi.LOOP_STAGE_INPUTS])
+def test_dependency_ordered_blocks_see_their_predecessors(gpu, stage, graph):
+    """Many small blocks that share cache lines over all XCDs, run after run: a
+    block adds to what its predecessors wrote, never to an older value."""
+    p = airfoil_problem(110, 100, seed=3, block_size=32)
+    p.reorder("gps")
+    f = capi.functor(capi.KERNEL_RES_CALC)
+    dev = [DeviceArray.from_host(d) for d in p.point_data]
+    out = DeviceArray.from_host(np.zeros_like(p.point_data[0]))
+    got = []
+    for flags in (stage, stage | capi.LOOP_DEPENDENCY_ORDER):
+        loop = Loop(f, p.maps, p.num_points, dev, out, (), block_size=32, flags=flags,
+                    use_graph=graph)
+        for _ in range(1 if flags == stage else 400):
+            dev[0].upload(p.point_data[0])
+            loop.run(2)
+            got.append(dev[0].download())
+        loop.close()
+    for i, g in enumerate(got[1:]):
+        assert_bitwise(g, got[0], f"run {i}")
